@@ -309,101 +309,117 @@ __device__ __forceinline__ float grid_sample(const GridDev& g, V3 p, V3 plq, V3&
     return E;
 }
 
-// The same sample with the atom's 4x4x4 window of channel-combined
-// coefficients (cs = plq . c, 64 floats = 256 B) kept in a per-atom cache
-// slot in global memory.  While the atom stays in the same grid cell (the
-// window base `key` is unchanged) the 64 gathers from the 10 MB grid become
-// one contiguous 256 B read that stays in L2; on a cell change the window is
-// gathered, combined and written back.  Same arithmetic as grid_sample.
-// Cubic B-spline basis value and derivative of index a (0..3) at u: the
-// slab loop below runs rolled, so the four weights are computed per slab.
-__device__ __forceinline__ void bs_basis_a(float u, int a, float& b, float& d) {
+// Basis values and derivatives of one axis for grid_sample_wave, every
+// rounding written out (fused where __builtin_fmaf stands, nowhere else).
+__device__ __forceinline__ void bs_weights(float u, float* b, float* d) {
+#pragma clang fp contract(off)
     const float inv6 = 1.f / 6.f;
     const float u2 = u * u;
     const float t = 1.f - u;
-    switch (a) {
-        case 0: b = inv6 * t * t * t; d = -0.5f * t * t; break;
-        case 1: b = inv6 * (3.f * u2 * (u - 2.f) + 4.f); d = 0.5f * (3.f * u2 - 4.f * u); break;
-        case 2: b = inv6 * (3.f * u * (1.f + u - u2) + 1.f); d = 0.5f * (-3.f * u2 + 2.f * u + 1.f); break;
-        default: b = inv6 * u2 * u; d = 0.5f * u2; break;
-    }
+    const float q = 3.f * u2;
+    b[0] = t * (t * (inv6 * t));
+    b[1] = inv6 * __builtin_fmaf(u - 2.f, q, 4.f);
+    b[2] = inv6 * __builtin_fmaf(3.f * u, __builtin_fmaf(-u, u, u + 1.f), 1.f);
+    b[3] = u * (inv6 * u2);
+    d[0] = t * (-0.5f * t);
+    d[1] = 0.5f * __builtin_fmaf(-4.f, u, q);
+    d[2] = 0.5f * (__builtin_fmaf(2.f, u, -q) + 1.f);
+    d[3] = 0.5f * u2;
 }
 
-__device__ __forceinline__ float grid_sample_cached(const GridDev& g, V3 p, V3 plq, float4* cache, int stride, int& key,
-                                                    V3& f) {
-    const float ux = (p.x - g.p0x) * g.isx;
-    const float uy = (p.y - g.p0y) * g.isy;
-    const float uz = (p.z - g.p0z) * g.isz;
-    int ix = (int)ux, iy = (int)uy, iz = (int)uz;
+// The same sample for the atoms of a whole wave (every lane calls; `act` marks
+// the lanes with an atom) through a cache in global memory: each atom owns a
+// slot of 16 float4 with the 4x4x4 window of channel-combined coefficients
+// cs = plq . c, row r = a*4+b of atom `lane` at cache[r*stride + lane].  While
+// an atom stays in the grid cell of its slot (window base `key`) the 64 gathers
+// from the 10 MB grid become one read of the slot, which stays in L2.
+//
+// A step moves a few of a wave's 64 atoms across a cell face (0.1 A), so nearly
+// every step refills some slots.  A refill is done by the whole wave: lane l
+// fetches coefficient (a, b, c) = (l>>4, (l>>2)&3, l&3) of the leaving atom's new
+// window, one load instruction of 16 runs of 64 B, and stores its combined value
+// into the slot.  Refilling in the atom's own lane instead takes 64 loads in a
+// row with one or two lanes active, and was 60-80 % of this function's time.
+// Reads of the slots follow the stores of the same wave in program order.
+__device__ __forceinline__ void grid_sample_wave(const GridDev& g, bool act, V3 p, V3 plq, float4* cache, int stride,
+                                                 int& key, V3& f) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63;
+    const float qx = p.x - g.p0x, qy = p.y - g.p0y, qz = p.z - g.p0z;
+    const float ux = qx * g.isx, uy = qy * g.isy;
+    int ix = (int)ux, iy = (int)uy, iz = (int)(qz * g.isz);
     if (ux < 0.f) ix--;
     if (uy < 0.f) iy--;
-    const float tx = ux - ix, ty = uy - iy, tz = uz - iz;
+    const float tx = __builtin_fmaf(g.isx, qx, -(float)ix);
+    const float ty = __builtin_fmaf(g.isy, qy, -(float)iy);
+    const float tz = __builtin_fmaf(g.isz, qz, -(float)iz);
     iz = min(max(iz, 3), g.nz - 5);
     ix = imod(ix - 1, g.nx);
     iy = imod(iy - 1, g.ny);
     const int k = (ix * g.ny + iy) * g.nz + iz;
-    const bool hit = (k == key);
-    key = k;
-    float by[4], dy[4], bz[4], dz[4];
-    bs_basis(ty, by);
-    bs_dbasis(ty, dy);
-    bs_basis(tz, bz);
-    bs_dbasis(tz, dz);
-    float Fx = 0.f, Fy = 0.f, Fz = 0.f, E = 0.f;
-#pragma unroll 1
-    for (int a = 0; a < 4; a++) {  // x-slabs one at a time: 16 coefficients live
-        float cs[16];
-        if (hit) {
+    unsigned long long miss = __ballot(act && k != key);
+    key = act ? k : key;
+    if (miss) {
+        const int la = lane >> 4, lb = (lane >> 2) & 3, lc = (lane & 3) - 1;
+        float* slot = reinterpret_cast<float*>(cache + (size_t)(lane >> 2) * stride) + (lane & 3);
+        do {
+            // up to four atoms' loads in flight at once
+            int m[4];
+            float4 q[4];
+            const int n = min((int)__popcll(miss), 4);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float4 v = cache[(a * 4 + q) * stride];
-                cs[q * 4 + 0] = v.x;
-                cs[q * 4 + 1] = v.y;
-                cs[q * 4 + 2] = v.z;
-                cs[q * 4 + 3] = v.w;
-            }
-        } else {
-            int xa = ix + a;
-            if (xa >= g.nx) xa -= g.nx;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                int yb = iy + b;
-                if (yb >= g.ny) yb -= g.ny;
-                const float4* col = g.coefs + ((size_t)(xa * g.ny + yb) * g.nz + (iz - 1));
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const float4 q = col[c];
-                    cs[b * 4 + c] = plq.x * q.x + plq.y * q.y + plq.z * q.z;
-                }
+            for (int t = 0; t < 4; t++) {
+                if (t >= n) break;
+                m[t] = (int)__ffsll(miss) - 1;
+                miss &= miss - 1;
+                int xa = __builtin_amdgcn_readlane(ix, m[t]) + la;
+                int yb = __builtin_amdgcn_readlane(iy, m[t]) + lb;
+                xa = min((unsigned)xa, (unsigned)(xa - g.nx));  // periodic: 0 <= xa < nx + 3
+                yb = min((unsigned)yb, (unsigned)(yb - g.ny));
+                q[t] = g.coefs[(size_t)(xa * g.ny + yb) * g.nz + (__builtin_amdgcn_readlane(iz, m[t]) + lc)];
             }
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                cache[(a * 4 + q) * stride] = make_float4(cs[q * 4], cs[q * 4 + 1], cs[q * 4 + 2], cs[q * 4 + 3]);
-        }
+            for (int t = 0; t < 4; t++) {
+                if (t >= n) break;
+                auto bcast = [&](float v) {
+                    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), m[t]));
+                };
+                const float cx = bcast(plq.x), cy = bcast(plq.y), cz = bcast(plq.z);
+                slot[m[t] * 4] = __builtin_fmaf(cz, q[t].z, __builtin_fmaf(cx, q[t].x, cy * q[t].y));
+            }
+        } while (miss);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    const float4* mine = cache + (act ? lane : 0);  // lane 0 has an atom
+    float bx[4], dx[4], by[4], dy[4], bz[4], dz[4];
+    bs_weights(tx, bx, dx);
+    bs_weights(ty, by, dy);
+    bs_weights(tz, bz, dz);
+    float Fx = 0.f, Fy = 0.f, Fz = 0.f;
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
         float ey = 0.f, fy = 0.f, fz = 0.f;
 #pragma unroll
         for (int b = 0; b < 4; b++) {
-            float e = 0.f, de = 0.f;
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                e += bz[c] * cs[b * 4 + c];
-                de += dz[c] * cs[b * 4 + c];
-            }
-            fy += e * dy[b];
-            fz += de * by[b];
-            ey += e * by[b];
+            const float4 cs = mine[(a * 4 + b) * stride];
+            float e = __builtin_fmaf(bz[0], cs.x, 0.f), de = __builtin_fmaf(dz[0], cs.x, 0.f);
+            e = __builtin_fmaf(bz[1], cs.y, e);
+            de = __builtin_fmaf(dz[1], cs.y, de);
+            e = __builtin_fmaf(bz[2], cs.z, e);
+            de = __builtin_fmaf(dz[2], cs.z, de);
+            e = __builtin_fmaf(bz[3], cs.w, e);
+            de = __builtin_fmaf(dz[3], cs.w, de);
+            fy = __builtin_fmaf(dy[b], e, fy);
+            fz = __builtin_fmaf(by[b], de, fz);
+            ey = __builtin_fmaf(by[b], e, ey);
         }
-        float bxa, dxa;
-        bs_basis_a(tx, a, bxa, dxa);
-        Fx += ey * dxa;
-        Fy += fy * bxa;
-        Fz += fz * bxa;
-        E += ey * bxa;
+        Fx = __builtin_fmaf(ey, dx[a], Fx);
+        Fy = __builtin_fmaf(fy, bx[a], Fy);
+        Fz = __builtin_fmaf(fz, bx[a], Fz);
     }
-    f.x -= Fx * g.isx;
-    f.y -= Fy * g.isy;
-    f.z -= Fz * g.isz;
-    return E;
+    f.x = __builtin_fmaf(-g.isx, Fx, f.x);
+    f.y = __builtin_fmaf(-g.isy, Fy, f.y);
+    f.z = __builtin_fmaf(-g.isz, Fz, f.z);
 }
 
 // -------------------------------------------------------------------------

@@ -388,12 +388,11 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                                 f -= d * (fr * pc.w);
                             }
                         }
-                        if (P.bGridFF) {
-                            grid_sample_cached(P.grid, pi, mk(plq.x, plq.y, plq.z), B.gridcache + I.a0 + i,
-                                               B.gridcache_stride, gkey, f);
-                        }
-                        s_fnb[i] = make_float4(f.x, f.y, f.z, 0.f);
                     }
+                    if (P.bGridFF && wu < nwAct)  // the atoms of a wave together
+                        grid_sample_wave(P.grid, hasAtom, pi, mk(plq.x, plq.y, plq.z), B.gridcache + I.a0 + wu * 64,
+                                         B.gridcache_stride, gkey, f);
+                    if (hasAtom) s_fnb[tid] = make_float4(f.x, f.y, f.z, 0.f);
                     if (hasNode) {
                         V3 fbs[4], fps[4], fa, fpi;
                         auto pos = [&](int v) { return xyz(s_pos[v]); };
