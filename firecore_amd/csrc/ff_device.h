@@ -34,6 +34,25 @@ __device__ __forceinline__ float dpp_shl1_zero(float src) {
                                                                  true));
 }
 
+// Stores v at LDS byte address `addr` + off (off a constant) from lane 0 alone;
+// all lanes call with exec full.  Narrowing exec for one instruction costs two
+// scalar ones; the branch the compiler makes of `if (lane == 0)` costs six and
+// splits the block, so nothing is scheduled across it.
+typedef float f32x3 __attribute__((ext_vector_type(3)));
+#define lane0_store(addr, off, v)                                                                          \
+    asm volatile("s_mov_b64 exec, 1\n\tds_write_b96 %0, %1 offset:%2\n\ts_mov_b64 exec, -1" ::"v"(addr), \
+                 "v"(f32x3{(v).x, (v).y, (v).z}), "n"(off)                                                 \
+                 : "memory")
+
+// All ones where bit BIT of w is set, else 0 (one instruction; as C++ the and
+// with it becomes an and, a compare and a select).
+template <int BIT>
+__device__ __forceinline__ int lane_mask(unsigned w) {
+    int r;
+    asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(r) : "v"(w), "n"(BIT));
+    return r;
+}
+
 // Switches of the bonded terms (setSwitches_multi, MMFFmulti_lib.cpp:316-329).
 struct FFSwitch {
     int doBonds, doPiPiI, doPiSigma, doAngles;
@@ -220,6 +239,25 @@ __device__ __forceinline__ void lj_pair(V3 d, float Rij, float Eij, float kQQ, f
         e = Eq + (u6 - 2.f) * vdW;
         fr = (Eq + (u6 - 1.f) * vdW * 12.f) * ir2;
     }
+}
+
+// Force factor of lj_pair<HB> alone (force on i = d * -fr), every rounding
+// written out.
+template <bool HB>
+__device__ __forceinline__ float lj_force(V3 d, float Rij, float Eij, float kQQ, float Hij) {
+#pragma clang fp contract(off)
+    const float r2 = __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.x, d.x, d.y * d.y));
+    const float ir = __builtin_amdgcn_rsqf(r2);
+    const float ir2 = ir * ir;
+    const float u2 = (Rij * Rij) * ir2;
+    const float u4 = u2 * u2;
+    const float u6 = u2 * u4;
+    const float vdW = Eij * u6;
+    const float t = __builtin_fmaf(u2, u4, -1.f);
+    float s;
+    if (HB) s = __builtin_fmaf(t, vdW, ((Hij < 0.f) ? Eij * Hij : 0.f) * (u6 * u6));
+    else s = t * vdW;
+    return __builtin_fmaf(kQQ, ir, s * 12.f) * ir2;
 }
 
 // -------------------------------------------------------------------------

@@ -70,11 +70,19 @@ __device__ __forceinline__ void mlp_features(V3 F, V3 G, V3 p, V3 Fb, int elem, 
     x[15] = 0.1f * height;
 }
 
+// Bonded neighbours of a row: an int4 (as packed) or the short4 that the
+// relaxation kernel keeps in LDS (local indices fit 16 bits there).
+__device__ __forceinline__ int4 nb_row(const int4* nb, int i) { return nb[i]; }
+__device__ __forceinline__ int4 nb_row(const short4* nb, int i) {
+    const short4 q = nb[i];
+    return make_int4(q.x, q.y, q.z, q.w);
+}
+
 // A operand of row block rb, K chunk kc from the activation rows in LDS.
 // Chunks 0..KS-1 read the atom's own row; chunks KS.. read the sum over its
 // bonded neighbours (FP32 sum of bf16 rows, rounded to bf16).
-template <int KS>
-__device__ __forceinline__ bf16x4 mlp_a_frag(const unsigned short* h, const int4* nb, int n, int rb, int kc,
+template <int KS, class NB>
+__device__ __forceinline__ bf16x4 mlp_a_frag(const unsigned short* h, const NB* nb, int n, int rb, int kc,
                                              int lane) {
     const int row = rb * 16 + (lane & 15);
     const int kk = 4 * (lane >> 4);
@@ -89,7 +97,7 @@ __device__ __forceinline__ bf16x4 mlp_a_frag(const unsigned short* h, const int4
         a[2] = (short)(u.y & 0xFFFFu);
         a[3] = (short)(u.y >> 16);
     } else {
-        const int4 n4 = (row < n) ? nb[row] : make_int4(-1, -1, -1, -1);
+        const int4 n4 = (row < n) ? nb_row(nb, row) : make_int4(-1, -1, -1, -1);
         const int ns[4] = {n4.x, n4.y, n4.z, n4.w};
         float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
 #pragma unroll
@@ -113,7 +121,8 @@ __device__ __forceinline__ bf16x4 mlp_a_frag(const unsigned short* h, const int4
 // row l%16, K values 8*(l/16)..+7 of the chunk): chunks 0,1 are the atom's own
 // row (64 columns), chunks 2,3 the bf16-rounded FP32 sum over its bonded
 // neighbours, element by element as in mlp_a_frag.
-__device__ __forceinline__ bf16x8 mlp_a_frag32(const unsigned short* h, const int4* nb, int n, int rb, int kc,
+template <class NB>
+__device__ __forceinline__ bf16x8 mlp_a_frag32(const unsigned short* h, const NB* nb, int n, int rb, int kc,
                                                int lane) {
     const int row = rb * 16 + (lane & 15);
     const int kk = 8 * (lane >> 4);
@@ -132,7 +141,7 @@ __device__ __forceinline__ bf16x8 mlp_a_frag32(const unsigned short* h, const in
         a[6] = (short)(u1.y & 0xFFFFu);
         a[7] = (short)(u1.y >> 16);
     } else {
-        const int4 n4 = (row < n) ? nb[row] : make_int4(-1, -1, -1, -1);
+        const int4 n4 = (row < n) ? nb_row(nb, row) : make_int4(-1, -1, -1, -1);
         const int ns[4] = {n4.x, n4.y, n4.z, n4.w};
         float sm[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -301,8 +310,8 @@ __device__ __forceinline__ void mlp_forward(const MlpDev& M, unsigned short* h, 
 // row buffers of n rows, hA (LDS) and hG (LDS when the workgroup's LDS budget
 // allows, else a per-workgroup slot in global memory that stays in L2):
 // layer 1 hA -> hG, layer 2 hG -> hA, layer 3 hA -> hG, head from hG.
-template <int BLOCK, int KIN>
-__device__ __forceinline__ void mlp_layer_rows(const unsigned short* hin, const int4* nb, const unsigned short* W,
+template <int BLOCK, int KIN, class NB>
+__device__ __forceinline__ void mlp_layer_rows(const unsigned short* hin, const NB* nb, const unsigned short* W,
                                                const float* bias, int n, unsigned short* hout) {
     constexpr int NW = BLOCK / 64;
     constexpr int NK = KIN / 16;
@@ -371,9 +380,9 @@ __device__ __forceinline__ void mlp_layer_rows(const unsigned short* hin, const 
 // returns the two head outputs of row threadIdx.x (zeros for threads >= n).
 // The global writes of a layer are made visible to the whole workgroup by
 // the fence + barrier that follow them.
-template <int BLOCK>
+template <int BLOCK, class NB>
 __device__ __forceinline__ float2 mlp_forward_rows(const MlpDev& M, unsigned short* hA, unsigned short* hG,
-                                                   const int4* nb, int n) {
+                                                   const NB* nb, int n) {
     mlp_layer_rows<BLOCK, 16>(hA, nb, M.W1, M.b1, n, hG);
     __threadfence_block();
     __syncthreads();
@@ -401,8 +410,10 @@ __device__ __forceinline__ float2 mlp_forward_rows(const MlpDev& M, unsigned sho
 // Feature row of atom i (bf16, columns 0..15 of its activation row).  F is
 // the exact atom force, G its substrate part (recomputed here), pi the atom's
 // pi-vector (nodes only), Fb the mean exact force of its bonded neighbours.
-__device__ __forceinline__ void mlp_feature_row(const RunParams& P, const float4* s_pos, const float4* s_F,
-                                                const int4* nb, const int* elem, int N, int M, int i, float4 plq,
+// s_pi: the pi-vectors of the nodes.
+__device__ __forceinline__ void mlp_feature_row(const RunParams& P, const float4* s_pos, const float4* s_pi,
+                                                const float4* s_F,
+                                                const int4* nb, const int* elem, int M, int i, float4 plq,
                                                 unsigned short* hrow, const V3* Gpre = nullptr) {
     const V3 p = xyz(s_pos[i]);
     V3 G = zero3();
@@ -419,7 +430,7 @@ __device__ __forceinline__ void mlp_feature_row(const RunParams& P, const float4
             deg++;
         }
     if (deg) Fb = Fb * (1.f / (float)deg);
-    const V3 pi = (i < M) ? xyz(s_pos[N + i]) : zero3();
+    const V3 pi = (i < M) ? xyz(s_pi[i]) : zero3();
     const float height = P.bGridFF ? p.z - P.grid.p0z : 0.f;
     float x[MLP_NIN];
     mlp_features(xyz(s_F[i]), G, pi, Fb, elem[i], deg, i < M, height, x);
@@ -433,24 +444,23 @@ __device__ __forceinline__ void mlp_feature_row(const RunParams& P, const float4
 // receives per-wave partial sums (component output sums and atom counts).
 // Every thread calls it; nothing of the step loop is live across the call.
 template <int BLOCK>
-__device__ __forceinline__ void propose_gains(const RunParams& P, const int4* nb, const float4* req, const int* elem,
-                              const float4* s_pos, const float4* s_F, float4* s_req, unsigned short* h,
+__device__ __forceinline__ void propose_gains(const RunParams& P, const int4* nb, const int* elem,
+                              const float4* s_pos, const float4* s_pi, const float4* s_F, short4* s_nb, unsigned short* h,
                               unsigned short* hG, float* s_gain, float* s_cred, int N, int M, int nc, int myc,
                               float4 plq) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wid = tid >> 6;
     constexpr int NW = BLOCK / 64;
-    // the bonded neighbour lists are read for every operand fragment: stage
-    // them in LDS over the (constant) REQ rows, restored from req below
-    int4* s_nb = reinterpret_cast<int4*>(s_req);
+    // the bonded neighbour lists are read for every operand fragment: they are
+    // staged in LDS in s_nb
     if (tid < N) {
-        mlp_feature_row(P, s_pos, s_F, nb, elem, N, M, tid, plq, h + tid * MLP_HS);
-        s_nb[tid] = nb[tid];
+        mlp_feature_row(P, s_pos, s_pi, s_F, nb, elem, M, tid, plq, h + tid * MLP_HS);
+        const int4 q = nb[tid];
+        s_nb[tid] = make_short4((short)q.x, (short)q.y, (short)q.z, (short)q.w);
     }
     __syncthreads();
     const float2 o = mlp_forward_rows<BLOCK>(P.mlp, h, hG, s_nb, N);
-    if (tid < N) s_req[tid] = req[tid];
     if (tid < M) s_gain[tid] = P.pc_gstar * sigmoidf_(o.x);
     for (int c = 0; c < nc; c++) {
         const bool mine = tid < N && myc == c;

@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(256) k_train_fwd(BatchDev B, RunParams P, Trai
     __syncthreads();
     if (tid < N) {
         unsigned short* hrow = s_h + tid * MLP_HS;
-        mlp_feature_row(P, s_pos, s_F, B.neighs + I.a0, B.elem + I.a0, N, M, tid, B.PLQs[I.a0 + tid], hrow);
+        mlp_feature_row(P, s_pos, s_pos + N, s_F, B.neighs + I.a0, B.elem + I.a0, M, tid, B.PLQs[I.a0 + tid], hrow);
 #pragma unroll
         for (int k = 0; k < MLP_NIN; k++) T.X[(size_t)(I.a0 + tid) * MLP_NIN + k] = hrow[k];
     }
@@ -497,7 +497,7 @@ __global__ void __launch_bounds__(256) k_mlp_gains(BatchDev B, RunParams P, floa
     if (tid < N) s_F[tid] = B.aforce[I.v0 + tid];
     __syncthreads();
     if (tid < N)
-        mlp_feature_row(P, s_pos, s_F, B.neighs + I.a0, B.elem + I.a0, N, M, tid, B.PLQs[I.a0 + tid],
+        mlp_feature_row(P, s_pos, s_pos + N, s_F, B.neighs + I.a0, B.elem + I.a0, M, tid, B.PLQs[I.a0 + tid],
                         s_h + tid * MLP_HS);
     __syncthreads();
     mlp_forward<BLOCK>(P.mlp, s_h, B.neighs + I.a0, N, s_out, nullptr, nullptr);

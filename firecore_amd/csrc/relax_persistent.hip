@@ -29,39 +29,53 @@
 
 namespace fcd {
 
-template <int BLOCK>
-struct BlockRed {
-    static constexpr int NW = BLOCK / 64;
-};
+// Four small signed indices (atoms, or recoil rows: below 2048) in two registers.
+__device__ __forceinline__ uint2 pack4(int4 a) {
+    return make_uint2(((unsigned)a.x & 0xFFFFu) | ((unsigned)a.y << 16), ((unsigned)a.z & 0xFFFFu) | ((unsigned)a.w << 16));
+}
+__device__ __forceinline__ int4 unpack4(uint2 p) {
+    return make_int4((int)(short)p.x, (int)p.x >> 16, (int)(short)p.y, (int)p.y >> 16);
+}
 
 // LDS layout (bytes), computed identically on the host (world.cpp).
-//   pos   float4[nmax+mmax]     positions of atoms and pi-vectors
-//   req   float4[nmax]          (R0, sqrt(E0), Q, H)
+//   pos   float4[prow+mmax]     (x, y, z, Q) of the atoms as periodic rows: row r
+//                              holds atom r mod N, so the partners of an atom at
+//                              offsets 0..N/2 follow it without a wrap; then the
+//                              pi-vectors, from row prow
+//   re    float2[prow]          (R0, sqrt(E0)) in the same rows
+//   hb    float[prow]           H of the same rows (batches with H-bond charges)
 //   fnb   float4[nmax]          non-bonded + grid force accumulated by atom i's thread
 //   facc  float4[nwave*frow]    per-wave reaction forces of the half-ring schedule:
-//                              wave w's row holds partners 64w+1 .. 64w+63+nmax/2
+//                              entry e of wave w's row is the reaction on atom
+//                              (64w+e) mod N
 //   fself float4[2*mmax]        bonded self forces of nodes and pi-vectors
 //   fng   float4[8*mmax]        recoils (sigma rows, then pi rows)
-//   mask  uint[wmax*nmax]       rotated exclusion rows, [word][atom]; only the
-//                              words of offsets k <= nmax/2 (wmax = nmax/64 + 1)
+//   mask  uint[wmax*nmax]       rotated exclusion rows, [word][atom]: the whole words
+//                              below the one of the last offset, which each
+//                              thread keeps in a register
 //   learned gains only:
 //   gain  float[mmax+PC_MAXC]   gains of the stars and the components
 //   h     bf16 rows            network activations (one of the two buffers),
 //                              aliased onto facc..mask, which is padded to fit
 struct LdsLayout {
-    int nmax, mmax, wmax, nwave, learned, h2lds;
+    int nmax, mmax, nwave, learned, h2lds, hb;
     __host__ __device__ static int r16(int b) { return (b + 15) & ~15; }
-    __host__ __device__ int vmax() const { return nmax + mmax; }
+    // rows the pair loop reads: offsets 0..N/2, rounded up to whole iterations, and
+    // the next iteration's first rows read ahead
+    __host__ __device__ static int prow_of(int n) { return n + (n >> 1) + 8; }
+    __host__ __device__ int prow() const { return prow_of(nmax); }
+    __host__ __device__ int wmax() const { return nmax >> 6; }
     __host__ __device__ int off_pos() const { return 0; }
-    __host__ __device__ int off_req() const { return off_pos() + vmax() * 16; }
-    __host__ __device__ int off_fnb() const { return off_req() + nmax * 16; }
+    __host__ __device__ int off_re() const { return off_pos() + (prow() + mmax) * 16; }
+    __host__ __device__ int off_hb() const { return off_re() + r16(prow() * 8); }
+    __host__ __device__ int off_fnb() const { return off_hb() + (hb ? r16(prow() * 4) : 0); }
     __host__ __device__ int off_facc() const { return off_fnb() + nmax * 16; }
-    // entries of a wave's reaction row: lane l's partner at offset k lands at l+k-1
-    __host__ __device__ int frow() const { return 64 + (nmax >> 1); }
+    // entries of a wave's reaction row: lane l's partner at offset k lands at l+k
+    __host__ __device__ int frow() const { return 64 + (nmax >> 1) + 4; }
     __host__ __device__ int off_fself() const { return off_facc() + nwave * frow() * 16; }
     __host__ __device__ int off_fng() const { return off_fself() + 2 * mmax * 16; }
     __host__ __device__ int off_mask() const { return off_fng() + 8 * mmax * 16; }
-    __host__ __device__ int end_base() const { return off_mask() + nmax * wmax * 4; }
+    __host__ __device__ int end_base() const { return off_mask() + nmax * wmax() * 4; }
     __host__ __device__ int hbytes() const { return r16(nmax * MLP_HS * 2); }
     __host__ __device__ int off_gain() const {
         const int e = end_base();
@@ -105,7 +119,9 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
     extern __shared__ float4 lds_dyn[];
     char* lds = reinterpret_cast<char*>(lds_dyn);
     float4* s_pos = reinterpret_cast<float4*>(lds + L.off_pos());
-    float4* s_req = reinterpret_cast<float4*>(lds + L.off_req());
+    float4* s_pi = s_pos + L.prow();
+    float2* s_re = reinterpret_cast<float2*>(lds + L.off_re());
+    float* s_hb = reinterpret_cast<float*>(lds + L.off_hb());
     float4* s_fnb = reinterpret_cast<float4*>(lds + L.off_fnb());
     float4* s_fself = reinterpret_cast<float4*>(lds + L.off_fself());
     float4* s_fng = reinterpret_cast<float4*>(lds + L.off_fng());
@@ -158,8 +174,10 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
         const SysInfo I = B.info[s];
         const int N = I.natoms, M = I.nnode, V = N + M;
         const int sflags = B.sysflags ? B.sysflags[s] : 0;  // restraints (bit 0), walls (bit 1)
-        const int W = (N + 31) >> 5;         // exclusion words per atom in memory
-        const int Wh = ((N >> 1) >> 5) + 1;  // words of the offsets k <= N/2 the half ring reads
+        const int W = (N + 31) >> 5;   // exclusion words per atom in memory
+        const int Kl = N >> 1;         // last offset of the half ring
+        const int Wh = Kl >> 5;        // its exclusion word, kept in a register; the words below it are in LDS
+        const int PR = LdsLayout::prow_of(N);  // periodic rows of this system
         // exclusion rows transposed to [word][atom] so that lanes read consecutive banks
         auto stage_mask = [&] {
             for (int w = tid; w < N * Wh; w += BLOCK) {
@@ -167,10 +185,28 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                 s_mask[wd * N + a] = B.excl_rot[I.mask0 + a * W + wd];
             }
         };
+        auto stage_re = [&] {
+            for (int r = tid; r < PR; r += BLOCK) {
+                const float4 q = B.REQs[I.a0 + r % N];
+                s_re[r] = make_float2(q.x, q.y);
+                if (HB) s_hb[r] = q.w;
+            }
+        };
+        // row of vec v in s_pos, and the parameters of atom j as they were given
+        auto vrow = [&](int v) { return v < N ? v : L.prow() + v - N; };
+        auto req = [&](int j) {
+            const float2 q = s_re[j];
+            return make_float4(q.x, q.y, s_pos[j].w, HB ? s_hb[j] : 0.f);
+        };
 
         // ---- stage the system in LDS
-        for (int v = tid; v < V; v += BLOCK) s_pos[v] = B.atoms[I.v0 + v];
-        for (int i = tid; i < N; i += BLOCK) s_req[i] = B.REQs[I.a0 + i];
+        for (int r = tid; r < PR; r += BLOCK) {
+            const int a = r % N;
+            const float4 p = B.atoms[I.v0 + a];
+            s_pos[r] = make_float4(p.x, p.y, p.z, B.REQs[I.a0 + a].z);
+        }
+        for (int k = tid; k < M; k += BLOCK) s_pi[k] = B.atoms[I.v0 + N + k];
+        stage_re();
         stage_mask();
 
         const bool hasAtom = tid < N;
@@ -258,36 +294,49 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
             bool propose_now = false;
             // ---- per-thread state of this segment: atom tid, node tid, vecs tid and tid+BLOCK
             const float4 plq = hasAtom ? B.PLQs[I.a0 + tid] : make_float4(0, 0, 0, 0);
+            // exclusion word of the half ring's last offset
+            const unsigned mlast = hasAtom ? B.excl_rot[I.mask0 + tid * W + Wh] : 0u;
             const int myc = (PC && hasAtom) ? B.comp[I.a0 + tid] : 0;
-            int4 ng = make_int4(-1, -1, -1, -1);
+            uint2 ngp = pack4(make_int4(-1, -1, -1, -1));
             float4 apar = make_float4(0, 0, 0, 0), bL = apar, bK = apar, ksp = apar, kpp = apar;
             if (hasNode) {
-                ng = B.neighs[I.a0 + tid];
+                ngp = pack4(B.neighs[I.a0 + tid]);
                 apar = B.apars[I.n0 + tid];
                 bL = B.bLs[I.n0 + tid];
                 bK = B.bKs[I.n0 + tid];
                 ksp = B.Ksp[I.n0 + tid];
                 kpp = B.Kpp[I.n0 + tid];
             }
-            int4 bk[2];
+            uint2 bkp[2];
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 const int v = tid + r * BLOCK;
-                bk[r] = make_int4(-1, -1, -1, -1);
+                bkp[r] = pack4(make_int4(-1, -1, -1, -1));
                 if (v < V) {
                     // back-neighbours as local indices into s_fng (sigma rows [0,4M), pi rows [4M,8M))
-                    int4 b = B.bkNeighs[I.v0 + v];
+                    const int4 b = B.bkNeighs[I.v0 + v];
                     const int base = I.n0 * 8;
-                    bk[r].x = b.x >= 0 ? b.x - base : -1;
-                    bk[r].y = b.y >= 0 ? b.y - base : -1;
-                    bk[r].z = b.z >= 0 ? b.z - base : -1;
-                    bk[r].w = b.w >= 0 ? b.w - base : -1;
+                    bkp[r] = pack4(make_int4(b.x >= 0 ? b.x - base : -1, b.y >= 0 ? b.y - base : -1,
+                                             b.z >= 0 ? b.z - base : -1, b.w >= 0 ? b.w - base : -1));
                 }
             }
             for (;;) {
+                // The compiler would hoist everything a step derives from these out of
+                // the loop and spill it; opaque copies keep it inside.
+                int tid_ = tid;
+                asm volatile("" : "+v"(tid_), "+v"(ngp.x), "+v"(ngp.y), "+v"(bkp[0].x), "+v"(bkp[0].y), "+v"(bkp[1].x),
+                             "+v"(bkp[1].y));
+                const int tid = tid_;
+                const int lane = tid & 63;
+                const int wid = tid >> 6;
+                const bool hasAtom = tid < N;
+                const bool hasNode = tid < M;
                 if (B.snap && step % B.snap_every == 0 && step / B.snap_every < B.nsnap) {
                     float4* dst = B.snap + (size_t)(step / B.snap_every) * B.ntotV + I.v0;
-                    for (int v = tid; v < V; v += BLOCK) dst[v] = s_pos[v];
+                        for (int v = tid; v < V; v += BLOCK) {
+                        const float4 p = s_pos[vrow(v)];
+                        dst[v] = make_float4(p.x, p.y, p.z, 0.f);
+                    }
                 }
                 float vf = 0.f, vv = 0.f, ff = 0.f, fm2 = 0.f;
                 if (!fresh) {
@@ -299,38 +348,61 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     // by one atom per offset.  The reaction on each partner is accumulated
                     // in registers and moves down one lane per offset with the window
                     // (DPP wave shift; the atom entering at lane 63 starts from zero); the
-                    // reaction leaving at lane 0 is written to the wave's reaction row.
-                    // Entry e of wave w's row holds the reaction on atom (64w+1+e) mod N:
-                    // entries 0..N/2-2 are written as they leave, the rest by all 64 lanes
-                    // after the last offset.  Every entry is written once and read after
-                    // the block barrier: no clearing, no atomics, no lane ordering.
+                    // reaction leaving at lane 0 is written to the wave's reaction row:
+                    // entry k as it leaves, the last 64 by all lanes after the last
+                    // offset.  Every entry is written once and read after the block
+                    // barrier: no clearing, no atomics, no lane ordering.
+                    //
+                    // The loop is bound by VALU issue (4.6 cycles per instruction, three
+                    // resident waves per SIMD), so everything but the pair itself is kept
+                    // out of it.  Partners come from periodic rows at addresses that advance
+                    // by a constant (no index wrap); the exclusion bit of an offset becomes
+                    // a lane mask in one instruction and is applied in one; offsets are
+                    // taken four per iteration, two computed side by side, with the rows of
+                    // the next two on their way.  Offset 0 (an atom with itself) and the
+                    // offsets past N/2 that round up the last iteration are masked as
+                    // excluded pairs are.  31.5 instructions per offset; with wrapped
+                    // indices and one offset at a time it took 40, and waited for LDS.
                     const int nwAct = (N + 63) >> 6;
-                    const int Kl = N >> 1;          // last offset of the half ring
-                    const int nrow = 63 + Kl;       // entries of a wave's reaction row
+                    const int nrow = 64 + Kl;       // entries of a wave's reaction row that hold a reaction
                     const int wu = __builtin_amdgcn_readfirstlane(wid);
                     V3 f = zero3();
                     // lanes without an atom carry the window only: their own atom sits far
                     // away with zero parameters, so each of their pair forces is exactly 0
-                    const V3 pi = hasAtom ? xyz(s_pos[tid]) : mk(1e4f, 1e4f, 1e4f);
-                    const float4 ri = hasAtom ? s_req[tid] : make_float4(0.f, 0.f, 0.f, 0.f);
+                    const float4 p4 = s_pos[hasAtom ? tid : 0];
+                    const V3 pi = hasAtom ? xyz(p4) : mk(1e4f, 1e4f, 1e4f);
+                    float4 ri = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (hasAtom) ri = req(tid);
                     const float kQi = COULOMB_K * ri.z;
                     if (P.bNonBonded && wu < nwAct && N >= 2) {
-                        float4* facc = s_facc + wu * L.frow();
-                        const int ic = hasAtom ? tid : 0;
-                        unsigned j = (unsigned)((wu * 64 + lane + 1) % N);  // partner at offset 1
+                        const int ia = hasAtom ? tid : 0;
+                        const float4* pp = s_pos + ia;
+                        const float2* pr = s_re + ia;
+                        const float* ph = s_hb + ia;
                         V3 acc = zero3();
-                        // one offset: the pair (i, j) with partner rows (pj, rj), excluded when
-                        // bit k of the offset's mask word is set; reads the next offset's
-                        // partner rows into (pn, rn) ahead of the arithmetic
-                        auto pair_step = [&](unsigned mword, int k, const float4& pj, const float4& rj, float4& pn,
-                                             float4& rn) {
-                            j = min(j + 1, j + 1 - (unsigned)N);  // (j+1) mod N
-                            pn = s_pos[j];
-                            rn = s_req[j];
-                            const V3 d = mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
-                            float fr, ep;
-                            lj_pair<HB>(d, ri.x + rj.x, ri.y * rj.y, kQi * rj.z, ri.w * rj.w, fr, ep);
-                            fr = ((mword >> (k & 31)) & 1u) ? 0.f : fr;
+                        struct Rows {
+                            float4 p;
+                            float2 r;
+                            float h;
+                        };
+                        auto rows = [&](int k) {
+                            Rows q;
+                            q.p = pp[k];
+                            q.r = pr[k];
+                            q.h = HB ? ph[k] : 0.f;
+                            return q;
+                        };
+                        // address of the entry that leaves at the iteration's first offset
+                        unsigned fout = (unsigned)(size_t)(
+                            (__attribute__((address_space(3))) char*)(lds + L.off_facc() + wu * L.frow() * 16));
+                        // the pair with the rows q: force on the partner = d * fr
+                        auto pair = [&](const Rows& q, V3& d, float& fr) {
+                            d = mk(q.p.x - pi.x, q.p.y - pi.y, q.p.z - pi.z);
+                            fr = lj_force<HB>(d, ri.x + q.r.x, ri.y * q.r.y, kQi * q.p.w, ri.w * q.h);
+                        };
+                        // adds the pair, masked by bit `bit` of keep, and moves the window on
+                        auto add = [&](V3 d, float fr, int keep) {
+                            fr = __builtin_bit_cast(float, __builtin_bit_cast(int, fr) & keep);
                             f.x = __builtin_fmaf(-d.x, fr, f.x);
                             f.y = __builtin_fmaf(-d.y, fr, f.y);
                             f.z = __builtin_fmaf(-d.z, fr, f.z);
@@ -338,40 +410,58 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                             acc.y = __builtin_fmaf(d.y, fr, acc.y);
                             acc.z = __builtin_fmaf(d.z, fr, acc.z);
                         };
-                        // the window moves on: the reaction of lane 0's partner leaves
-                        auto shift = [&](int k) {
-                            if (lane == 0) facc[k - 1] = make_float4(acc.x, acc.y, acc.z, 0.f);
+                        auto shift = [&] {
                             acc.x = dpp_shl1_zero(acc.x);
                             acc.y = dpp_shl1_zero(acc.y);
                             acc.z = dpp_shl1_zero(acc.z);
                         };
-                        float4 pA = s_pos[j], rA = s_req[j], pB, rB;
-                        // offsets 1..Kl-1, two per iteration (partner rows alternate A/B)
-                        for (int w = 0; (w << 5) < Kl; w++) {
-                            const unsigned m = s_mask[w * N + ic];
-                            const int k0 = max(1, w << 5);
-                            const int k1 = min(Kl - 1, (w << 5) + 31);
-                            int k = k0;
-                            for (; k < k1; k += 2) {
-                                pair_step(m, k, pA, rA, pB, rB);
-                                shift(k);
-                                pair_step(m, k + 1, pB, rB, pA, rA);
-                                shift(k + 1);
+                        Rows a0 = rows(0), a1 = rows(1), b0, b1;
+                        unsigned keep = 0;
+                        const int Kn = (Kl & ~3) + 4;  // offsets taken: 0..Kn-1
+#pragma clang loop unroll(disable)
+                        for (int k = 0;; k += 4) {
+                            if ((k & 31) == 0) {  // the next exclusion word, as bits of the pairs to keep
+                                const int w = k >> 5;
+                                keep = ~(w < Wh ? s_mask[w * N + ia] : mlast);
+                                if (w == 0) keep &= ~1u;
+                                if (w == Wh) {  // nothing past N/2; for even N the pair at N/2 is the lower half's
+                                    const int top = (Kl & 31) + ((!(N & 1) && tid >= Kl) ? 0 : 1);
+                                    keep &= top < 32 ? (1u << top) - 1u : ~0u;
+                                }
                             }
-                            if (k == k1) {
-                                pair_step(m, k, pA, rA, pB, rB);
-                                shift(k);
-                                pA = pB;
-                                rA = rB;
-                            }
+                            pp += 2;
+                            pr += 2;
+                            ph += 2;
+                            b0 = rows(0);
+                            b1 = rows(1);
+                            V3 d0, d1;
+                            float g0, g1;
+                            pair(a0, d0, g0);
+                            pair(a1, d1, g1);
+                            add(d0, g0, lane_mask<0>(keep));
+                            lane0_store(fout, 0, acc);
+                            shift();
+                            add(d1, g1, lane_mask<1>(keep));
+                            lane0_store(fout, 16, acc);
+                            shift();
+                            pp += 2;
+                            pr += 2;
+                            ph += 2;
+                            a0 = rows(0);
+                            a1 = rows(1);
+                            pair(b0, d0, g0);
+                            pair(b1, d1, g1);
+                            add(d0, g0, lane_mask<2>(keep));
+                            lane0_store(fout, 32, acc);
+                            shift();
+                            add(d1, g1, lane_mask<3>(keep));
+                            if (k + 4 == Kn) break;
+                            lane0_store(fout, 48, acc);
+                            shift();
+                            keep >>= 4;
+                            fout += 64;
                         }
-                        // last offset Kl: for even N the pair (i, i+N/2) is taken by the lower half only
-                        {
-                            unsigned m = s_mask[(Kl >> 5) * N + ic];
-                            if (!(N & 1) && tid >= Kl) m |= 1u << (Kl & 31);
-                            pair_step(m, Kl, pA, rA, pB, rB);
-                        }
-                        facc[lane + Kl - 1] = make_float4(acc.x, acc.y, acc.z, 0.f);
+                        s_facc[wu * L.frow() + Kn - 1 + lane] = make_float4(acc.x, acc.y, acc.z, 0.f);
                     }
                     if (hasAtom) {
                         const int i = tid;
@@ -381,7 +471,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                                 const PairCorrDev pc = B.corr[I.corr0 + c];
                                 if (pc.i != i) continue;
                                 const float4 pj = s_pos[pc.j];
-                                const float4 rj = s_req[pc.j];
+                                const float4 rj = req(pc.j);
                                 const V3 d = mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
                                 float fr, ep;
                                 lj_pair<HB>(d, ri.x + rj.x, ri.y * rj.y, kQi * rj.z, ri.w * rj.w, fr, ep);
@@ -396,7 +486,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     if (hasNode) {
                         V3 fbs[4], fps[4], fa, fpi;
                         auto pos = [&](int v) { return xyz(s_pos[v]); };
-                        eval_node(tid, N, M, pos, ng, apar, bL, bK, ksp, kpp, P.sw, fbs, fps, fa, fpi);
+                        eval_node(tid, L.prow(), M, pos, unpack4(ngp), apar, bL, bK, ksp, kpp, P.sw, fbs, fps, fa, fpi);
 #pragma unroll
                         for (int k = 0; k < 4; k++) {
                             s_fng[tid * 4 + k] = make_float4(fbs[k].x, fbs[k].y, fbs[k].z, 0.f);
@@ -418,8 +508,8 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                             if (!isPi) {
                                 f = xyz(s_fnb[v]);
                                 if (P.bNonBonded && N >= 2)
-                                    for (int w = 0; w < nwAct; w++) {  // atom v: entries (v-64w-1) mod N + multiples of N
-                                        int e = (v - 64 * w - 1) % N;
+                                    for (int w = 0; w < nwAct; w++) {  // atom v: entries (v-64w) mod N + multiples of N
+                                        int e = v - 64 * w;            // > -N: an active wave's first atom is below N
                                         e = (e < 0) ? e + N : e;
                                         const float4* row = s_facc + w * L.frow();
                                         for (; e < nrow; e += N) f += xyz(row[e]);
@@ -433,14 +523,15 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                             } else {
                                 f = xyz(s_fself[M + (v - N)]);
                             }
-                            const int b4[4] = {bk[r].x, bk[r].y, bk[r].z, bk[r].w};
+                            const int4 b = unpack4(bkp[r]);
+                            const int b4[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
                             for (int k = 0; k < 4; k++) {
                                 if (b4[k] < 0) break;
                                 f += xyz(s_fng[b4[k]]);
                             }
                             if (isPi) {
-                                const V3 p = xyz(s_pos[v]);
+                                const V3 p = xyz(s_pi[v - N]);
                                 f -= p * dot(p, f);
                             }
                             fm2 = fmaxf(fm2, dot(f, f));  // convergence always on the exact force
@@ -483,7 +574,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                 }
                 if (PC)
                     precondition<BLOCK>(P, s_pos, s_fnb, s_fself, s_fng, &s_cred[0][0][0], &s_csum[0][0], s_gain,
-                                        learned, N, M, nc, myc, hasAtom, hasNode, ng, bk[0], fv[0]);
+                                        learned, N, M, nc, myc, hasAtom, hasNode, unpack4(ngp), unpack4(bkp[0]), fv[0]);
                 // FIRE sums: totals per chunk of 64 consecutive vecs (vec v = tid + r*BLOCK
                 // lies in chunk wid + r*NW), added in chunk order, so that the result does
                 // not depend on the workgroup width a system is relaxed with
@@ -529,17 +620,15 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     if (hasAtom && P.bNonBonded) {
                         const int i = tid;
                         const V3 pi = xyz(s_pos[i]);
-                        const float4 ri = s_req[i];
+                        const float4 ri = req(i);
                         const float kQi = COULOMB_K * ri.z;
                         double e = 0.0;  // each unordered pair once (half ring)
-                        const int Kh = N >> 1;
-                        for (int k = 1; k <= Kh; k++) {
-                            if (!(N & 1) && k == Kh && i >= Kh) break;
-                            if ((s_mask[(k >> 5) * N + i] >> (k & 31)) & 1u) continue;
-                            int j = i + k;
-                            j = (j >= N) ? j - N : j;
-                            const float4 pj = s_pos[j];
-                            const float4 rj = s_req[j];
+                        for (int k = 1; k <= Kl; k++) {
+                            if (!(N & 1) && k == Kl && i >= Kl) break;
+                            const unsigned mw = (k >> 5) < Wh ? s_mask[(k >> 5) * N + i] : mlast;
+                            if ((mw >> (k & 31)) & 1u) continue;
+                            const float4 pj = s_pos[i + k];
+                            const float4 rj = req(i + k);
                             float fr, ep;
                             lj_pair<true, true>(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), ri.x + rj.x, ri.y * rj.y,
                                                 kQi * rj.z, ri.w * rj.w, fr, ep);
@@ -550,7 +639,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                             const PairCorrDev pc = B.corr[I.corr0 + c];
                             if (pc.i != i) continue;
                             const float4 pj = s_pos[pc.j];
-                            const float4 rj = s_req[pc.j];
+                            const float4 rj = req(pc.j);
                             float fr, ep;
                             lj_pair<true, true>(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), ri.x + rj.x, ri.y * rj.y,
                                                 kQi * rj.z, ri.w * rj.w, fr, ep);
@@ -565,7 +654,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     if (hasNode) {
                         V3 fbs[4], fps[4], fa, fpi;
                         auto pos = [&](int v) { return xyz(s_pos[v]); };
-                        epart += (double)eval_node(tid, N, M, pos, ng, apar, bL, bK, ksp, kpp, P.sw, fbs, fps, fa, fpi);
+                        epart += (double)eval_node(tid, L.prow(), M, pos, unpack4(ngp), apar, bL, bK, ksp, kpp, P.sw, fbs, fps, fa, fpi);
                     }
                     double ed = wave_sum_d(epart);
                     if (lane == 0) s_redd[wid] = ed;
@@ -590,7 +679,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     const int v = tid + r * BLOCK;
                     if (v < V) {
                         const bool isPi = v >= N;
-                        V3 p = xyz(s_pos[v]);
+                        V3 p = xyz(s_pos[vrow(v)]);
                         V3 f = fv[r];
                         if (isPi) f -= p * dot(p, f);
                         V3 w = vel[r] * cv + f * (dt + cfe);
@@ -598,7 +687,14 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                         p += w * dt;
                         if (isPi) p = p * (1.f / sqrtf(dot(p, p)));
                         vel[r] = w;
-                        s_pos[v] = make_float4(p.x, p.y, p.z, 0.f);
+                        if (isPi) {
+                            s_pi[v - N] = make_float4(p.x, p.y, p.z, 0.f);
+                        } else {
+                            // the atom's periodic rows (two, more below 17 atoms); Q stays
+                            const f32x3 t = {p.x, p.y, p.z};
+                            *reinterpret_cast<f32x3*>(s_pos + v) = t;
+                            for (int q = v + N; q < PR; q += N) *reinterpret_cast<f32x3*>(s_pos + q) = t;
+                        }
                     }
                 }
                 step++;
@@ -613,10 +709,11 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                 if (v < V) B.avel[I.v0 + v] = make_float4(vel[r].x, vel[r].y, vel[r].z, 0.f);
             }
             __syncthreads();
-            propose_gains<BLOCK>(P, B.neighs + I.a0, B.REQs + I.a0, B.elem + I.a0, s_pos, s_fnb, s_req, s_h, g_h,
-                                 s_gain, &s_cred[0][0][0], N, M, nc, hasAtom ? B.comp[I.a0 + tid] : 0,
+            propose_gains<BLOCK>(P, B.neighs + I.a0, B.elem + I.a0, s_pos, s_pi, s_fnb,
+                                 reinterpret_cast<short4*>(s_re), s_h, g_h, s_gain, &s_cred[0][0][0], N, M, nc, hasAtom ? B.comp[I.a0 + tid] : 0,
                                  hasAtom ? B.PLQs[I.a0 + tid] : make_float4(0, 0, 0, 0));
-            stage_mask();  // the exclusion rows were overwritten by the activations
+            stage_mask();  // the exclusion rows were overwritten by the activations,
+            stage_re();    // the pair parameters by the neighbour lists
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 const int v = tid + r * BLOCK;
@@ -636,7 +733,10 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
         for (int r = 0; r < 2; r++) {
             const int v = tid + r * BLOCK;
             if (v < V) {
-                B.atoms[I.v0 + v] = s_pos[v];
+                if (step > 0) {  // else nothing has moved
+                    const float4 p = s_pos[vrow(v)];
+                    B.atoms[I.v0 + v] = make_float4(p.x, p.y, p.z, 0.f);
+                }
                 B.avel[I.v0 + v] = make_float4(vel[r].x, vel[r].y, vel[r].z, 0.f);
                 // preconditioned forms keep the exact atom forces in s_fnb; a suspended
                 // chunk holds them, assembled and not yet preconditioned, in fv
@@ -694,8 +794,8 @@ static const void* kernel_ptr(int block, int hb, int pc) {
 extern "C" hipError_t fc_launch_relax_persistent(int block, int hb, int ngroups, size_t lds_bytes, hipStream_t stream,
                                                  const fcd::BatchDev* B, const fcd::RunParams* P, const int* order,
                                                  const int* qinfo, int* counters, int cls, int nmax, int mmax,
-                                                 int wmax, int steal, unsigned short* hslot, int h2lds) {
-    fcd::LdsLayout L{nmax, mmax, wmax, block / 64, P->pc_mode == 2 ? 1 : 0, h2lds};
+                                                 int steal, unsigned short* hslot, int h2lds) {
+    fcd::LdsLayout L{nmax, mmax, block / 64, P->pc_mode == 2 ? 1 : 0, h2lds, hb};
     fcd::Queues Q;
     Q.order = order;
     for (int c = 0; c < 4; c++) {
@@ -738,14 +838,14 @@ extern "C" hipError_t fc_noalloc_scratch(void** ptr) {
     return hipSuccess;
 }
 
-extern "C" int fc_lds_bytes(int nmax, int mmax, int wmax, int block, int learned, int h2lds) {
-    fcd::LdsLayout L{nmax, mmax, wmax, block / 64, learned, h2lds};
+extern "C" int fc_lds_bytes(int nmax, int mmax, int block, int learned, int h2lds, int hb) {
+    fcd::LdsLayout L{nmax, mmax, block / 64, learned, h2lds, hb};
     return L.bytes();
 }
 
 // bf16 elements of one workgroup's global activation slot (the second buffer)
 extern "C" int fc_hslot_elems(int nmax) {
-    fcd::LdsLayout L{nmax, 1, 1, 1, 1, 0};
+    fcd::LdsLayout L{nmax, 1, 1, 1, 0, 0};
     return L.hbytes() / 2;
 }
 

@@ -53,7 +53,7 @@ extern "C" hipError_t fc_launch_zero_f4(hipStream_t st, float4* a, int n);
 extern "C" hipError_t fc_launch_relax_persistent(int block, int hb, int ngroups, size_t lds_bytes, hipStream_t stream,
                                                  const fcd::BatchDev* B, const fcd::RunParams* P, const int* order,
                                                  const int* qinfo, int* counters, int cls, int nmax, int mmax,
-                                                 int wmax, int steal, unsigned short* hslot, int h2lds);
+                                                 int steal, unsigned short* hslot, int h2lds);
 
 namespace fcw {
 
@@ -231,7 +231,7 @@ int World::relax_learned(int nstep_max, double Fconv, bool restore_start) {
             hipStream_t cs = class_streams[k % class_streams.size()];
             hipStreamWaitEvent(cs, evs[0], 0);
             if (!hip_ok(fc_launch_relax_persistent(C.block, hb_batch ? 1 : 0, C.ngroups, C.lds, cs, &B, &P, d_order.p,
-                                                   qinfo.data(), d_queue.p, C.cls, C.nmax, C.mmax, C.wmax,
+                                                   qinfo.data(), d_queue.p, C.cls, C.nmax, C.mmax,
                                                    sched_mode == 0 ? 1 : 0, nullptr, 0),
                         "relax chunk"))
                 return false;

@@ -17,12 +17,12 @@
 extern "C" hipError_t fc_launch_relax_persistent(int block, int hb, int ngroups, size_t lds_bytes, hipStream_t stream,
                                                  const fcd::BatchDev* B, const fcd::RunParams* P, const int* order,
                                                  const int* qinfo, int* counters, int cls, int nmax, int mmax,
-                                                 int wmax, int steal, unsigned short* hslot, int h2lds);
+                                                 int steal, unsigned short* hslot, int h2lds);
 extern "C" int fc_hslot_elems(int nmax);
 extern "C" hipError_t fc_noalloc_scratch(void** ptr);
 extern "C" hipError_t fc_launch_zero_int(hipStream_t st, int* a, int n);
 extern "C" hipError_t fc_launch_zero_f4(hipStream_t st, float4* a, int n);
-extern "C" int fc_lds_bytes(int nmax, int mmax, int wmax, int block, int learned, int h2lds);
+extern "C" int fc_lds_bytes(int nmax, int mmax, int block, int learned, int h2lds, int hb);
 extern "C" hipError_t fc_launch_split_step(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P,
                                            const int* node_sys, int ntot_nodes, int maxN, int do_move, int step);
 extern "C" hipError_t fc_launch_reset(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P);
@@ -685,16 +685,15 @@ void World::plan_classes(bool upload) {
         mrun = std::max(mrun, C.mmax);
         C.nmax = nrun;
         C.mmax = mrun;
-        C.wmax = ((C.nmax >> 1) >> 5) + 1;  // exclusion words of the offsets k <= nmax/2
         // learned gains: the second activation buffer goes to LDS when the class
         // keeps two resident workgroups per CU pair of SIMDs (see plan below)
         C.h2lds = 0;
-        C.lds = (size_t)fc_lds_bytes(std::max(C.nmax, 1), std::max(C.mmax, 1), std::max(C.wmax, 1), C.block,
-                                     pc_mode == 2 ? 1 : 0, 0);
+        C.lds = (size_t)fc_lds_bytes(std::max(C.nmax, 1), std::max(C.mmax, 1), C.block, pc_mode == 2 ? 1 : 0, 0,
+                                     hb_batch ? 1 : 0);
         if (pc_mode == 2 && h2lds_allowed) {
             const size_t budget = (size_t)160 * 1024 / std::max(1, 8 / (C.block / 64));
-            const size_t with = (size_t)fc_lds_bytes(std::max(C.nmax, 1), std::max(C.mmax, 1), std::max(C.wmax, 1),
-                                                     C.block, 1, 1);
+            const size_t with = (size_t)fc_lds_bytes(std::max(C.nmax, 1), std::max(C.mmax, 1), C.block, 1, 1,
+                                                     hb_batch ? 1 : 0);
             if (with <= budget) {
                 C.h2lds = 1;
                 C.lds = with;
@@ -791,7 +790,7 @@ int World::relax_persistent(int nstep_max, double Fconv, bool restore_start) {
         hipEvent_t es = events.make(), ev = events.make();
         hipEventRecord(es, st);
         hipError_t err = fc_launch_relax_persistent(C.block, hb_batch ? 1 : 0, C.ngroups, C.lds, st, &B, &P, d_order.p,
-                                                    qinfo.data(), d_queue.p, C.cls, C.nmax, C.mmax, C.wmax,
+                                                    qinfo.data(), d_queue.p, C.cls, C.nmax, C.mmax,
                                                     sched_mode == 0 ? 1 : 0,
                                                     pc_mode == 2 ? d_hslot.p + slot_off[k] : nullptr, C.h2lds);
         if (!hip_ok(err, "relax_persistent launch")) return -1;
@@ -886,7 +885,7 @@ int World::relax_noalloc(int nstep_max, double Fconv, bool restore_start) {
         hipStream_t st = class_streams[k % class_streams.size()];
         hipStreamWaitEvent(st, fork, 0);
         hipError_t err = fc_launch_relax_persistent(C.block, hb_batch ? 1 : 0, C.ngroups, C.lds, st, &B, &P, order,
-                                                    qinfo.data(), counters, C.cls, C.nmax, C.mmax, C.wmax,
+                                                    qinfo.data(), counters, C.cls, C.nmax, C.mmax,
                                                     sched_mode == 0 ? 1 : 0, pc_mode == 2 ? hslot + slot_off[k] : nullptr,
                                                     C.h2lds);
         if (!hip_ok(err, "relax_noalloc launch")) return -1;

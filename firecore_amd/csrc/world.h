@@ -44,7 +44,7 @@ struct SizeClass {
     int block = 256;
     int cls = 0;   // index among the four widths (queue index)
     int occ = 1;   // resident workgroups per CU
-    int nmax = 0, mmax = 0, wmax = 0;
+    int nmax = 0, mmax = 0;
     std::vector<int> order;  // system indices, decreasing cost
     double work = 0;         // sum of N^2
     int ngroups = 0;
