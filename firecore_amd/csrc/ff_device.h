@@ -27,6 +27,23 @@ __device__ __forceinline__ V3 cross(V3 a, V3 b) {
     return V3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 
+// The thread index as a value that the compiler cannot see through.  It hoists
+// whatever derives from threadIdx.x (LDS and global addresses, masks, unpacked
+// neighbour lists) out of the relaxation kernel's loops and then spills it: with an
+// index of its own per system, segment and step the kernel needs 30 registers fewer.
+__device__ __forceinline__ int opaque_tid() {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
+// Gives v some value without an instruction.  A variable that is set on some paths
+// only counts as carried from iteration to iteration, and holds its registers all
+// the time; set to anything on the other paths it does not.
+__device__ __forceinline__ void any_value(float4& v) {
+    asm volatile("" : "=v"(v.x), "=v"(v.y), "=v"(v.z), "=v"(v.w));
+}
+
 // Wave shift by one lane (DPP wave_shl:1 with bound_ctrl): lane l receives
 // lane l+1's value, lane 63 receives 0.  Needs all 64 lanes active.
 __device__ __forceinline__ float dpp_shl1_zero(float src) {
@@ -207,6 +224,102 @@ __device__ __forceinline__ float eval_node(int ia, int natoms, int nnode, PosFn 
                      fpi);
 }
 
+// Forces of eval_node for a vacuum molecule in LDS (pi-vector of node k at
+// pos(pi0 + k)), without branches and without the energy: the neighbours are read at
+// once, the four neighbours' norms and then the angles two by two run side by side,
+// where the branches of eval_node wait for each read, root and division in turn (5800
+// cycles a step for a wave of nodes, a third of them issuing).  Terms that a node does
+// not have are computed on a unit vector and weighted zero.  The roundings are those
+// that the compiler gives eval_node, written out.  put_pi(i, f) takes the recoil on
+// neighbour i's pi-vector.  With the window reads below spread over the step, a system of
+// 251 atoms takes 24.0 us a step instead of 25.4 (constant gains), and 512 molecules on
+// the grid are scanned in 4.73 ms instead of 5.3.
+template <class PosFn, class PutPi>
+__device__ __forceinline__ void node_forces(int ia, int pi0, int nnode, PosFn pos, const int4 ng, const float4 apar,
+                                            const float4 bL, const float4 bK, const float4 ksp, const float4 kpp,
+                                            const FFSwitch sw, PutPi put_pi, V3* fbs, V3& fa, V3& fpi) {
+#pragma clang fp contract(off)
+    auto madd = [](V3 a, float k, V3 c) {
+        return mk(__builtin_fmaf(a.x, k, c.x), __builtin_fmaf(a.y, k, c.y), __builtin_fmaf(a.z, k, c.z));
+    };
+    // computed here and not put off until the end, which would keep all operands
+    auto now = [](V3& a) { asm volatile("" : "+v"(a.x), "+v"(a.y), "+v"(a.z)); };
+    auto dotp = [](V3 a, V3 b) { return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.x, b.x, a.y * b.y)); };
+    const int ings[4] = {ng.x, ng.y, ng.z, ng.w};
+    const float bLs[4] = {bL.x, bL.y, bL.z, bL.w};
+    const float bKs[4] = {bK.x, bK.y, bK.z, bK.w};
+    const float Ksp[4] = {ksp.x, ksp.y, ksp.z, ksp.w};
+    const float Kpp[4] = {kpp.x, kpp.y, kpp.z, kpp.w};
+    bool has[4];
+    V3 hs[4];
+    float l[4], ir[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        has[i] = (i == 0 || has[i - 1]) && ings[i] >= 0;
+        hs[i] = pos(has[i] ? ings[i] : ia);
+    }
+    const V3 pa = pos(ia);
+    const V3 hpi = pos(pi0 + ia);
+    fa = zero3();
+    fpi = zero3();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        V3 h = mk(hs[i].x - pa.x, hs[i].y - pa.y, hs[i].z - pa.z);
+        h = mk(has[i] ? h.x : 1.f, has[i] ? h.y : 0.f, has[i] ? h.z : 0.f);
+        l[i] = sqrtf(dotp(h, h));
+        ir[i] = 1.f / l[i];
+        hs[i] = mk(h.x * ir[i], h.y * ir[i], h.z * ir[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const V3 h = hs[i];
+        const bool first = has[i] && ia < ings[i];
+        const bool pin = has[i] && ings[i] < nnode;
+        const V3 hp = pos(pi0 + (pin ? ings[i] : ia));
+        float fr = (l[i] - bLs[i]) * bKs[i];  // bond
+        fr = (first && sw.doBonds) ? fr : 0.f;
+        fbs[i] = madd(h, -fr, zero3());
+        fa = madd(h, fr, fa);
+        float c = dotp(hpi, hp);  // pi-pi
+        float k = (first && pin && sw.doPiPiI && Kpp[i] > 1e-6f) ? Kpp[i] : 0.f;
+        k = c < 0.f ? -k : k;
+        fpi = madd(madd(hpi, -c, hp), k, fpi);
+        put_pi(i, madd(madd(hp, -c, hpi), k, zero3()));
+        c = dotp(hpi, h);  // pi-sigma
+        k = (has[i] && sw.doPiSigma && Ksp[i] > 1e-6f) ? Ksp[i] : 0.f;
+        const float t = (c - apar.w) * -k;
+        const float fang = t + t;
+        const V3 f2 = madd(h, -c, hpi);
+        fpi = madd(madd(hpi, -c, h), fang, fpi);
+        fa = madd(f2, -(fang * ir[i]), fa);
+        fbs[i] = madd(f2, fang * ir[i], fbs[i]);
+        now(fa);
+        now(fpi);
+        now(fbs[i]);
+    }
+#pragma unroll
+    for (int p = 0; p < 6; p++) {
+        const int i = p < 3 ? 0 : (p < 5 ? 1 : 2), j = p < 3 ? p + 1 : (p < 5 ? p - 1 : 3);
+        const V3 h = hs[i] + hs[j];
+        const float d = __builtin_fmaf(h.z, h.z, __builtin_fmaf(h.y, h.y, h.x * h.x));
+        const float c2 = d * 0.25f;
+        const float s2 = __builtin_fmaf(d, -0.25f, 1.f) + 1e-14f;
+        const float c = sqrtf(c2);
+        const float s = sqrtf(s2);
+        const float csy = __builtin_fmaf(apar.y, c, -(apar.x * s));
+        float fr = (csy * -apar.z) / ((4.f * c) * s);
+        fr = (has[j] && sw.doAngles) ? fr : 0.f;
+        const float fr1 = fr * ir[i], fr2 = fr * ir[j];
+        const float a1 = -2.f * c2 * fr1, a2 = -2.f * c2 * fr2;
+        const V3 f1 = madd(h, fr1, mk(hs[i].x * a1, hs[i].y * a1, hs[i].z * a1));
+        const V3 f2 = madd(h, fr2, mk(hs[j].x * a2, hs[j].y * a2, hs[j].z * a2));
+        fa -= f1 + f2;
+        fbs[i] += f1;
+        fbs[j] += f2;
+        if (p & 1) now(fa);
+    }
+}
+
 // -------------------------------------------------------------------------
 // Directed non-bonded pair, Forces.h:341-360 (getLJQH): bare Coulomb, LJ and
 // the H-bond correction; REQ mixing Forces.h:270 (_mixREQ).  d = pj - pi;
@@ -270,6 +383,7 @@ struct GridDev {
     int nx, ny, nz;
     float p0x, p0y, p0z;
     float isx, isy, isz;  // 1/step
+    float rnx, rny;       // 1/nx, 1/ny (relaxation kernel)
 };
 
 __device__ __forceinline__ void bs_basis(float u, float* b) {
@@ -292,6 +406,16 @@ __device__ __forceinline__ void bs_dbasis(float u, float* d) {
 __device__ __forceinline__ int imod(int i, int m) {
     int r = i % m;
     return r < 0 ? r + m : r;
+}
+
+// imod for the whole wave, rm = 1/m: below 2^22 the quotient from a float reciprocal is
+// off by one at most (a third of the instructions of an integer division).
+__device__ __forceinline__ int imod_near(int i, int m, float rm) {
+    if (__any(i >= (1 << 22) || i <= -(1 << 22))) return imod(i, m);
+    int r = i - (int)((float)i * rm) * m;
+    r = r < 0 ? r + m : r;
+    r = r < 0 ? r + m : r;
+    return r >= m ? r - m : r;
 }
 
 // Returns E; adds the force to f.  plq = (cP, cL, cQ) of the atom.
@@ -347,7 +471,7 @@ __device__ __forceinline__ float grid_sample(const GridDev& g, V3 p, V3 plq, V3&
     return E;
 }
 
-// Basis values and derivatives of one axis for grid_sample_wave, every
+// Basis values and derivatives of one axis for GridWave, every
 // rounding written out (fused where __builtin_fmaf stands, nowhere else).
 __device__ __forceinline__ void bs_weights(float u, float* b, float* d) {
 #pragma clang fp contract(off)
@@ -366,99 +490,154 @@ __device__ __forceinline__ void bs_weights(float u, float* b, float* d) {
 }
 
 // The same sample for the atoms of a whole wave (every lane calls; `act` marks
-// the lanes with an atom) through a cache in global memory: each atom owns a
-// slot of 16 float4 with the 4x4x4 window of channel-combined coefficients
-// cs = plq . c, row r = a*4+b of atom `lane` at cache[r*stride + lane].  While
-// an atom stays in the grid cell of its slot (window base `key`) the 64 gathers
-// from the 10 MB grid become one read of the slot, which stays in L2.
+// the lanes with an atom, lane 0 among them) through a cache in global memory:
+// each atom owns a slot of 16 float4 with the 4x4x4 window of channel-combined
+// coefficients cs = plq . c, row r = a*4+b of the wave's n atoms at cache[r*n ..].
+// The wave's slots are one run of 256 n bytes.  While an atom stays in the grid cell
+// of its slot (window base `key`) the 64 gathers from the 10 MB grid become one read
+// of the slot.
 //
 // A step moves a few of a wave's 64 atoms across a cell face (0.1 A), so nearly
 // every step refills some slots.  A refill is done by the whole wave: lane l
 // fetches coefficient (a, b, c) = (l>>4, (l>>2)&3, l&3) of the leaving atom's new
 // window, one load instruction of 16 runs of 64 B, and stores its combined value
 // into the slot.  Refilling in the atom's own lane instead takes 64 loads in a
-// row with one or two lanes active, and was 60-80 % of this function's time.
+// row with one or two lanes active, and was 60-80 % of the sample's time.
 // Reads of the slots follow the stores of the same wave in program order.
-__device__ __forceinline__ void grid_sample_wave(const GridDev& g, bool act, V3 p, V3 plq, float4* cache, int stride,
-                                                 int& key, V3& f) {
-#pragma clang fp contract(off)
-    const int lane = threadIdx.x & 63;
-    const float qx = p.x - g.p0x, qy = p.y - g.p0y, qz = p.z - g.p0z;
-    const float ux = qx * g.isx, uy = qy * g.isy;
-    int ix = (int)ux, iy = (int)uy, iz = (int)(qz * g.isz);
-    if (ux < 0.f) ix--;
-    if (uy < 0.f) iy--;
-    const float tx = __builtin_fmaf(g.isx, qx, -(float)ix);
-    const float ty = __builtin_fmaf(g.isy, qy, -(float)iy);
-    const float tz = __builtin_fmaf(g.isz, qz, -(float)iz);
-    iz = min(max(iz, 3), g.nz - 5);
-    ix = imod(ix - 1, g.nx);
-    iy = imod(iy - 1, g.ny);
-    const int k = (ix * g.ny + iy) * g.nz + iz;
-    unsigned long long miss = __ballot(act && k != key);
-    key = act ? k : key;
-    if (miss) {
+//
+// The calls are spread over the force phase so that no wave waits for memory:
+// locate() starts the gathers of the first four leaving atoms before the bonded
+// terms, refill() stores them after, and each half of the slot is read by fetch()
+// before half of the pair loop and used by add() after it (a whole slot in flight
+// would take 64 registers).
+struct GridWave {
+    V3 t = {};   // position in the cell
+    int ix = 0, iy = 0, iz = 0;
+    unsigned long long miss = 0;  // lanes whose slot holds another window
+    int n0 = 0;  // gathers in flight from locate()
+    float4 q0[4];
+    float4 w[8];
+    V3 F = {};   // sum over the window
+
+    __device__ __forceinline__ GridWave() {
+#pragma unroll
+        for (int t = 0; t < 4; t++) any_value(q0[t]);
+    }
+    // starts the gathers of the first (up to B) atoms in `miss`; returns their number
+    template <int B>
+    __device__ __forceinline__ int gather(const GridDev& g, int lane, float4* q) {
         const int la = lane >> 4, lb = (lane >> 2) & 3, lc = (lane & 3) - 1;
-        float* slot = reinterpret_cast<float*>(cache + (size_t)(lane >> 2) * stride) + (lane & 3);
-        do {
-            // up to four atoms' loads in flight at once
-            int m[4];
-            float4 q[4];
-            const int n = min((int)__popcll(miss), 4);
+        const int n = min((int)__popcll(miss), B);
+        unsigned long long left = miss;
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                if (t >= n) break;
-                m[t] = (int)__ffsll(miss) - 1;
-                miss &= miss - 1;
-                int xa = __builtin_amdgcn_readlane(ix, m[t]) + la;
-                int yb = __builtin_amdgcn_readlane(iy, m[t]) + lb;
-                xa = min((unsigned)xa, (unsigned)(xa - g.nx));  // periodic: 0 <= xa < nx + 3
-                yb = min((unsigned)yb, (unsigned)(yb - g.ny));
-                q[t] = g.coefs[(size_t)(xa * g.ny + yb) * g.nz + (__builtin_amdgcn_readlane(iz, m[t]) + lc)];
-            }
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                if (t >= n) break;
-                auto bcast = [&](float v) {
-                    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), m[t]));
-                };
-                const float cx = bcast(plq.x), cy = bcast(plq.y), cz = bcast(plq.z);
-                slot[m[t] * 4] = __builtin_fmaf(cz, q[t].z, __builtin_fmaf(cx, q[t].x, cy * q[t].y));
-            }
-        } while (miss);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    }
-    const float4* mine = cache + (act ? lane : 0);  // lane 0 has an atom
-    float bx[4], dx[4], by[4], dy[4], bz[4], dz[4];
-    bs_weights(tx, bx, dx);
-    bs_weights(ty, by, dy);
-    bs_weights(tz, bz, dz);
-    float Fx = 0.f, Fy = 0.f, Fz = 0.f;
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        float ey = 0.f, fy = 0.f, fz = 0.f;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const float4 cs = mine[(a * 4 + b) * stride];
-            float e = __builtin_fmaf(bz[0], cs.x, 0.f), de = __builtin_fmaf(dz[0], cs.x, 0.f);
-            e = __builtin_fmaf(bz[1], cs.y, e);
-            de = __builtin_fmaf(dz[1], cs.y, de);
-            e = __builtin_fmaf(bz[2], cs.z, e);
-            de = __builtin_fmaf(dz[2], cs.z, de);
-            e = __builtin_fmaf(bz[3], cs.w, e);
-            de = __builtin_fmaf(dz[3], cs.w, de);
-            fy = __builtin_fmaf(dy[b], e, fy);
-            fz = __builtin_fmaf(by[b], de, fz);
-            ey = __builtin_fmaf(by[b], e, ey);
+        for (int t = 0; t < B; t++) {
+            any_value(q[t]);
+            if (t >= n) continue;
+            const int m = (int)__ffsll(left) - 1;
+            left &= left - 1;
+            int xa = __builtin_amdgcn_readlane(ix, m) + la;
+            int yb = __builtin_amdgcn_readlane(iy, m) + lb;
+            xa = min((unsigned)xa, (unsigned)(xa - g.nx));  // periodic: 0 <= xa < nx + 3
+            yb = min((unsigned)yb, (unsigned)(yb - g.ny));
+            q[t] = g.coefs[(size_t)(xa * g.ny + yb) * g.nz + (__builtin_amdgcn_readlane(iz, m) + lc)];
         }
-        Fx = __builtin_fmaf(ey, dx[a], Fx);
-        Fy = __builtin_fmaf(fy, bx[a], Fy);
-        Fz = __builtin_fmaf(fz, bx[a], Fz);
+        return n;
     }
-    f.x = __builtin_fmaf(-g.isx, Fx, f.x);
-    f.y = __builtin_fmaf(-g.isy, Fy, f.y);
-    f.z = __builtin_fmaf(-g.isz, Fz, f.z);
-}
+    // stores the n gathered windows and takes their atoms out of `miss`
+    template <int B>
+    __device__ __forceinline__ void store(V3 plq, int lane, float4* cache, int stride, int n, const float4* q) {
+#pragma clang fp contract(off)
+        float* slot = reinterpret_cast<float*>(cache + (lane >> 2) * stride) + (lane & 3);
+#pragma unroll
+        for (int t = 0; t < B; t++) {
+            if (t >= n) break;
+            const int m = (int)__ffsll(miss) - 1;
+            miss &= miss - 1;
+            auto bcast = [&](float v) {
+                return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), m));
+            };
+            const float cx = bcast(plq.x), cy = bcast(plq.y), cz = bcast(plq.z);
+            slot[m * 4] = __builtin_fmaf(cz, q[t].z, __builtin_fmaf(cx, q[t].x, cy * q[t].y));
+        }
+    }
+    __device__ __forceinline__ void locate(const GridDev& g, int lane, bool act, V3 p, int& key) {
+#pragma clang fp contract(off)
+        const float qx = p.x - g.p0x, qy = p.y - g.p0y, qz = p.z - g.p0z;
+        const float ux = qx * g.isx, uy = qy * g.isy;
+        ix = (int)ux;
+        iy = (int)uy;
+        iz = (int)(qz * g.isz);
+        if (ux < 0.f) ix--;
+        if (uy < 0.f) iy--;
+        t = mk(__builtin_fmaf(g.isx, qx, -(float)ix), __builtin_fmaf(g.isy, qy, -(float)iy),
+               __builtin_fmaf(g.isz, qz, -(float)iz));
+        iz = min(max(iz, 3), g.nz - 5);
+        ix = imod_near(ix - 1, g.nx, g.rnx);
+        iy = imod_near(iy - 1, g.ny, g.rny);
+        const int k = (ix * g.ny + iy) * g.nz + iz;
+        miss = __ballot(act && k != key);
+        key = act ? k : key;
+        if (miss) n0 = gather<4>(g, lane, q0);
+    }
+    __device__ __forceinline__ void refill(const GridDev& g, int lane, V3 plq, float4* cache, int stride) {
+        F = zero3();
+        if (miss) {
+            store<4>(plq, lane, cache, stride, n0, q0);
+            while (miss) {
+                float4 q[8];
+                const int n = gather<8>(g, lane, q);
+                store<8>(plq, lane, cache, stride, n, q);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+    __device__ __forceinline__ void fetch(int lane, const float4* cache, int stride, int half) {
+        asm volatile("" : "+v"(lane));  // else the row addresses are kept over the pair loop
+        const float4* mine = cache + half * 8 * stride + lane;
+#pragma unroll
+        for (int r = 0; r < 8; r++) w[r] = mine[r * stride];
+    }
+    __device__ __forceinline__ void no_fetch() {
+#pragma unroll
+        for (int r = 0; r < 8; r++) any_value(w[r]);
+    }
+    // adds the x-slabs 2*half and 2*half+1 of the window
+    __device__ __forceinline__ void add(int half) {
+#pragma clang fp contract(off)
+        asm volatile("" : "+v"(t.x), "+v"(t.y), "+v"(t.z));  // else the 24 weights are kept over the pair loop
+        float bx[4], dx[4], by[4], dy[4], bz[4], dz[4];
+        bs_weights(t.x, bx, dx);
+        bs_weights(t.y, by, dy);
+        bs_weights(t.z, bz, dz);
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            float ey = 0.f, fy = 0.f, fz = 0.f;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const float4 cs = w[a * 4 + b];
+                float e = __builtin_fmaf(bz[0], cs.x, 0.f), de = __builtin_fmaf(dz[0], cs.x, 0.f);
+                e = __builtin_fmaf(bz[1], cs.y, e);
+                de = __builtin_fmaf(dz[1], cs.y, de);
+                e = __builtin_fmaf(bz[2], cs.z, e);
+                de = __builtin_fmaf(dz[2], cs.z, de);
+                e = __builtin_fmaf(bz[3], cs.w, e);
+                de = __builtin_fmaf(dz[3], cs.w, de);
+                fy = __builtin_fmaf(dy[b], e, fy);
+                fz = __builtin_fmaf(by[b], de, fz);
+                ey = __builtin_fmaf(by[b], e, ey);
+            }
+            const float b1 = half ? bx[a + 2] : bx[a], d1 = half ? dx[a + 2] : dx[a];
+            F.x = __builtin_fmaf(ey, d1, F.x);
+            F.y = __builtin_fmaf(fy, b1, F.y);
+            F.z = __builtin_fmaf(fz, b1, F.z);
+        }
+    }
+    __device__ __forceinline__ void finish(const GridDev& g, V3& f) const {
+        f.x = __builtin_fmaf(-g.isx, F.x, f.x);
+        f.y = __builtin_fmaf(-g.isy, F.y, f.y);
+        f.z = __builtin_fmaf(-g.isz, F.z, f.z);
+    }
+};
 
 // -------------------------------------------------------------------------
 // Positional restraint and bounding wall of one atom at p, the terms of the

@@ -73,10 +73,10 @@ struct BatchDev {
     // 0, snap_every, 2*snap_every, ... into snap[k * ntotV + v0 + v], k < nsnap
     float4* snap;
     int snap_every, nsnap, ntotV;
-    // per-atom GridFF window cache of the persistent kernel: 16 float4 per atom,
-    // row r of atom a at gridcache[r * gridcache_stride + a] (coalesced over atoms)
+    // GridFF window cache of the persistent kernel: 16 float4 per atom; the n <= 64
+    // atoms of a wave, starting at atom a of the batch, own the run
+    // gridcache[16a .. 16(a+n)), row r of the wave's atom l at 16a + r*n + l
     float4* gridcache;
-    int gridcache_stride;
     // positional restraints and bounding walls (updateAtomsMMFFf4,
     // relax_multi.cl:997-1009): per atom constr = (x, y, z, on if > 0) and
     // constrK = per-axis stiffness (negative = 0); per system bbox = 3 float4

@@ -185,7 +185,7 @@ __device__ __forceinline__ void precondition(const RunParams& P, const float4* s
                                              bool learned, int N, int M, int nc, int myc, bool hasAtom,
                                              bool hasNode, int4 ng, int4 bk0, V3& fv0) {
     constexpr int NW = BLOCK / 64;
-    const int tid = threadIdx.x;
+    const int tid = opaque_tid();
     const int lane = tid & 63;
     const int wid = tid >> 6;
     const V3 org = xyz(s_pos[0]);

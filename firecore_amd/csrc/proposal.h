@@ -316,7 +316,7 @@ __device__ __forceinline__ void mlp_layer_rows(const unsigned short* hin, const 
     constexpr int NW = BLOCK / 64;
     constexpr int NK = KIN / 16;
     constexpr int KS = (KIN == 16) ? 1 : 4;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int tid = opaque_tid(), lane = tid & 63, wid = tid >> 6;
     const int nrb = (n + 15) >> 4;
     // the weight fragments of all four column blocks are loaded once per layer
     // (one memory latency); a wave then takes whole row blocks, builds their A
@@ -392,7 +392,7 @@ __device__ __forceinline__ float2 mlp_forward_rows(const MlpDev& M, unsigned sho
     __threadfence_block();
     __syncthreads();
     float2 o = make_float2(0.f, 0.f);
-    const int i = threadIdx.x;
+    const int i = opaque_tid();
     if (i < n) {
         o = make_float2(M.b4[0], M.b4[1]);
         const unsigned short* q = hG + i * MLP_HS;
@@ -448,7 +448,7 @@ __device__ __forceinline__ void propose_gains(const RunParams& P, const int4* nb
                               const float4* s_pos, const float4* s_pi, const float4* s_F, short4* s_nb, unsigned short* h,
                               unsigned short* hG, float* s_gain, float* s_cred, int N, int M, int nc, int myc,
                               float4 plq) {
-    const int tid = threadIdx.x;
+    const int tid = opaque_tid();
     const int lane = tid & 63;
     const int wid = tid >> 6;
     constexpr int NW = BLOCK / 64;

@@ -146,12 +146,9 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
     __shared__ float s_st_best;       // FIRE fallback of the learned form (below)
     __shared__ int s_st_cnt, s_st_plain;
 
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wid = tid >> 6;
-
     int cc = cls;
     for (;;) {
+        const int tid = opaque_tid();
         if (tid == 0) {
             int q = -1;
             while (cc >= Q.lowest) {
@@ -180,13 +177,13 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
         const int PR = LdsLayout::prow_of(N);  // periodic rows of this system
         // exclusion rows transposed to [word][atom] so that lanes read consecutive banks
         auto stage_mask = [&] {
-            for (int w = tid; w < N * Wh; w += BLOCK) {
+            for (int w = opaque_tid(); w < N * Wh; w += BLOCK) {
                 const int a = w / Wh, wd = w - a * Wh;
                 s_mask[wd * N + a] = B.excl_rot[I.mask0 + a * W + wd];
             }
         };
         auto stage_re = [&] {
-            for (int r = tid; r < PR; r += BLOCK) {
+            for (int r = opaque_tid(); r < PR; r += BLOCK) {
                 const float4 q = B.REQs[I.a0 + r % N];
                 s_re[r] = make_float2(q.x, q.y);
                 if (HB) s_hb[r] = q.w;
@@ -209,8 +206,6 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
         stage_re();
         stage_mask();
 
-        const bool hasAtom = tid < N;
-        const bool hasNode = tid < M;
         const int nc = PC ? B.ncomp[s] : 0;
         V3 vel[2];
 #pragma unroll
@@ -255,8 +250,9 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
         }
         // called by every thread of the block with its own max|F|^2 at a proposal point
         auto stall_check = [&](float fm2t) {
+            const int tid = opaque_tid();
             fm2t = wave_max(fm2t);
-            if (lane == 0) s_smax[wid] = fm2t;
+            if ((tid & 63) == 0) s_smax[tid >> 6] = fm2t;
             __syncthreads();
             if (tid == 0) {
                 float m = s_smax[0];
@@ -278,7 +274,6 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
         __syncthreads();
 
         int status = ST_RUNNING;
-        float fmax2_last = 0.f;
         V3 fv[2];
         // The learned form evaluates the network between segments of the step
         // loop (one segment per proposal period): the step loop breaks out at a
@@ -292,48 +287,49 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
         bool fresh = learned && !inkernel && step > 0;
         for (;;) {
             bool propose_now = false;
+            const int tid = opaque_tid();
+            const bool hasAtom = tid < N;
             // ---- per-thread state of this segment: atom tid, node tid, vecs tid and tid+BLOCK
-            const float4 plq = hasAtom ? B.PLQs[I.a0 + tid] : make_float4(0, 0, 0, 0);
             // exclusion word of the half ring's last offset
             const unsigned mlast = hasAtom ? B.excl_rot[I.mask0 + tid * W + Wh] : 0u;
             const int myc = (PC && hasAtom) ? B.comp[I.a0 + tid] : 0;
             uint2 ngp = pack4(make_int4(-1, -1, -1, -1));
-            float4 apar = make_float4(0, 0, 0, 0), bL = apar, bK = apar, ksp = apar, kpp = apar;
-            if (hasNode) {
-                ngp = pack4(B.neighs[I.a0 + tid]);
-                apar = B.apars[I.n0 + tid];
-                bL = B.bLs[I.n0 + tid];
-                bK = B.bKs[I.n0 + tid];
-                ksp = B.Ksp[I.n0 + tid];
-                kpp = B.Kpp[I.n0 + tid];
-            }
+            if (tid < M) ngp = pack4(B.neighs[I.a0 + tid]);
+            // parameters of atom and node tid, read again for every step (while the step before
+            // reduces and moves): the pair loop and the preconditioner need the registers
+            float4 apar, bL, bK, ksp, kpp;
+            V3 plq;
+            auto load_params = [&](int k) {
+                const int n = max(I.n0 + min(k, M - 1), 0);  // some node's where there is none
+                apar = B.apars[n];
+                bL = B.bLs[n];
+                bK = B.bKs[n];
+                ksp = B.Ksp[n];
+                kpp = B.Kpp[n];
+                plq = xyz(B.PLQs[I.a0 + min(k, N - 1)]);
+            };
+            load_params(tid);
             uint2 bkp[2];
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 const int v = tid + r * BLOCK;
-                bkp[r] = pack4(make_int4(-1, -1, -1, -1));
-                if (v < V) {
-                    // back-neighbours as local indices into s_fng (sigma rows [0,4M), pi rows [4M,8M))
-                    const int4 b = B.bkNeighs[I.v0 + v];
-                    const int base = I.n0 * 8;
-                    bkp[r] = pack4(make_int4(b.x >= 0 ? b.x - base : -1, b.y >= 0 ? b.y - base : -1,
-                                             b.z >= 0 ? b.z - base : -1, b.w >= 0 ? b.w - base : -1));
-                }
+                // back-neighbours as local indices into s_fng (sigma rows [0,4M), pi rows [4M,8M))
+                int4 b = B.bkNeighs[I.v0 + min(v, V - 1)];
+                if (v >= V) b = make_int4(-1, -1, -1, -1);
+                const int base = I.n0 * 8;
+                bkp[r] = pack4(make_int4(b.x >= 0 ? b.x - base : -1, b.y >= 0 ? b.y - base : -1,
+                                         b.z >= 0 ? b.z - base : -1, b.w >= 0 ? b.w - base : -1));
             }
             for (;;) {
-                // The compiler would hoist everything a step derives from these out of
-                // the loop and spill it; opaque copies keep it inside.
-                int tid_ = tid;
-                asm volatile("" : "+v"(tid_), "+v"(ngp.x), "+v"(ngp.y), "+v"(bkp[0].x), "+v"(bkp[0].y), "+v"(bkp[1].x),
-                             "+v"(bkp[1].y));
-                const int tid = tid_;
+                const int tid = opaque_tid();
+                asm volatile("" : "+v"(ngp.x), "+v"(ngp.y), "+v"(bkp[0].x), "+v"(bkp[0].y), "+v"(bkp[1].x), "+v"(bkp[1].y));
                 const int lane = tid & 63;
                 const int wid = tid >> 6;
                 const bool hasAtom = tid < N;
                 const bool hasNode = tid < M;
                 if (B.snap && step % B.snap_every == 0 && step / B.snap_every < B.nsnap) {
                     float4* dst = B.snap + (size_t)(step / B.snap_every) * B.ntotV + I.v0;
-                        for (int v = tid; v < V; v += BLOCK) {
+                    for (int v = tid; v < V; v += BLOCK) {
                         const float4 p = s_pos[vrow(v)];
                         dst[v] = make_float4(p.x, p.y, p.z, 0.f);
                     }
@@ -374,16 +370,33 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     float4 ri = make_float4(0.f, 0.f, 0.f, 0.f);
                     if (hasAtom) ri = req(tid);
                     const float kQi = COULOMB_K * ri.z;
-                    if (P.bNonBonded && wu < nwAct && N >= 2) {
+                    const bool onGrid = P.bGridFF && wu < nwAct;  // the atoms of a wave together
+                    GridWave gw;
+                    if (onGrid) gw.locate(P.grid, lane, hasAtom, pi, gkey);
+                    if (hasNode) {
+                        V3 fbs[4], fa, fpi;
+                        auto pos = [&](int v) { return xyz(s_pos[v]); };
+                        auto put = [&](int row, V3 g) { s_fng[row] = make_float4(g.x, g.y, g.z, 0.f); };
+                        node_forces(tid, L.prow(), M, pos, unpack4(ngp), apar, bL, bK, ksp, kpp, P.sw,
+                                    [&](int k, V3 g) { put(4 * M + tid * 4 + k, g); }, fbs, fa, fpi);
+#pragma unroll
+                        for (int k = 0; k < 4; k++) put(tid * 4 + k, fbs[k]);
+                        s_fself[tid] = make_float4(fa.x, fa.y, fa.z, 0.f);
+                        s_fself[M + tid] = make_float4(fpi.x, fpi.y, fpi.z, 0.f);
+                    }
+                    float4* slots = B.gridcache + (size_t)(I.a0 + wu * 64) * 16;
+                    const int nslot = min(64, N - wu * 64);
+                    if (onGrid) gw.refill(P.grid, lane, plq, slots, nslot);
+                    if (wu < nwAct) {
                         const int ia = hasAtom ? tid : 0;
                         const float4* pp = s_pos + ia;
                         const float2* pr = s_re + ia;
                         const float* ph = s_hb + ia;
                         V3 acc = zero3();
                         struct Rows {
-                            float4 p;
-                            float2 r;
-                            float h;
+                            float4 p = {};
+                            float2 r = {};
+                            float h = 0.f;
                         };
                         auto rows = [&](int k) {
                             Rows q;
@@ -415,15 +428,25 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                             acc.y = dpp_shl1_zero(acc.y);
                             acc.z = dpp_shl1_zero(acc.z);
                         };
-                        Rows a0 = rows(0), a1 = rows(1), b0, b1;
+                        Rows a0, a1, b0, b1;
+                        a0 = rows(0);
+                        a1 = rows(1);
                         unsigned keep = 0;
                         const int Kn = (Kl & ~3) + 4;  // offsets taken: 0..Kn-1
+                        const int kmid = (Kn >> 3) << 2;
+                        if (onGrid) gw.fetch(hasAtom ? lane : 0, slots, nslot, 0);
+                        else gw.no_fetch();
 #pragma clang loop unroll(disable)
                         for (int k = 0;; k += 4) {
+                            if (k == kmid && onGrid) {
+                                gw.add(0);
+                                gw.fetch(hasAtom ? lane : 0, slots, nslot, 1);
+                            }
                             if ((k & 31) == 0) {  // the next exclusion word, as bits of the pairs to keep
                                 const int w = k >> 5;
                                 keep = ~(w < Wh ? s_mask[w * N + ia] : mlast);
                                 if (w == 0) keep &= ~1u;
+                                if (!P.bNonBonded) keep = 0;
                                 if (w == Wh) {  // nothing past N/2; for even N the pair at N/2 is the lower half's
                                     const int top = (Kl & 31) + ((!(N & 1) && tid >= Kl) ? 0 : 1);
                                     keep &= top < 32 ? (1u << top) - 1u : ~0u;
@@ -461,6 +484,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                             keep >>= 4;
                             fout += 64;
                         }
+                        if (onGrid) gw.add(1);
                         s_facc[wu * L.frow() + Kn - 1 + lane] = make_float4(acc.x, acc.y, acc.z, 0.f);
                     }
                     if (hasAtom) {
@@ -479,22 +503,8 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                             }
                         }
                     }
-                    if (P.bGridFF && wu < nwAct)  // the atoms of a wave together
-                        grid_sample_wave(P.grid, hasAtom, pi, mk(plq.x, plq.y, plq.z), B.gridcache + I.a0 + wu * 64,
-                                         B.gridcache_stride, gkey, f);
+                    if (onGrid) gw.finish(P.grid, f);
                     if (hasAtom) s_fnb[tid] = make_float4(f.x, f.y, f.z, 0.f);
-                    if (hasNode) {
-                        V3 fbs[4], fps[4], fa, fpi;
-                        auto pos = [&](int v) { return xyz(s_pos[v]); };
-                        eval_node(tid, L.prow(), M, pos, unpack4(ngp), apar, bL, bK, ksp, kpp, P.sw, fbs, fps, fa, fpi);
-#pragma unroll
-                        for (int k = 0; k < 4; k++) {
-                            s_fng[tid * 4 + k] = make_float4(fbs[k].x, fbs[k].y, fbs[k].z, 0.f);
-                            s_fng[4 * M + tid * 4 + k] = make_float4(fps[k].x, fps[k].y, fps[k].z, 0.f);
-                        }
-                        s_fself[tid] = make_float4(fa.x, fa.y, fa.z, 0.f);
-                        s_fself[M + tid] = make_float4(fpi.x, fpi.y, fpi.z, 0.f);
-                    }
                     __syncthreads();
 
                     // ================= B: assemble + reductions
@@ -594,6 +604,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     const float t = wave_sum4(pvf, pvv, pff, 0.f);  // lane l: total of value l >> 4
                     if ((lane & 15) == 0 && lane < 48) s_red[lane >> 4][wid + r * NW] = t;
                 }
+                load_params(tid);  // for the energy of this geometry or the next step's bonded terms
                 fm2 = wave_max(fm2);
                 if (lane == 0) s_red[3][wid] = fm2;
                 __syncthreads();
@@ -609,7 +620,6 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                 fm2 = s_red[3][0];
 #pragma unroll
                 for (int w = 1; w < NW; w++) fm2 = fmaxf(fm2, s_red[3][w]);
-                fmax2_last = fm2;
                 const float crit = (P.conv_mode == CONV_F2SUM) ? ff : fm2;
                 if (!(ff == ff) || isinf(ff)) status = ST_NAN;
                 else if (crit < P.Fconv2) status = ST_CONVERGED;
@@ -649,7 +659,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     }
                     if (hasAtom && P.bGridFF) {
                         V3 fd = zero3();
-                        epart += (double)grid_sample(P.grid, xyz(s_pos[tid]), mk(plq.x, plq.y, plq.z), fd);
+                        epart += (double)grid_sample(P.grid, xyz(s_pos[tid]), plq, fd);
                     }
                     if (hasNode) {
                         V3 fbs[4], fps[4], fa, fpi;
@@ -703,6 +713,9 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
             }
             if (!propose_now) break;
             // ---- network evaluation between segments (learned form)
+            {
+            const int tid = opaque_tid();
+            const bool hasAtom = tid < N;
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 const int v = tid + r * BLOCK;
@@ -719,10 +732,12 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                 const int v = tid + r * BLOCK;
                 if (v < V) vel[r] = xyz(B.avel[I.v0 + v]);
             }
+            }
             fresh = true;
             __syncthreads();
         }
-        (void)fmax2_last;
+        {
+        const int tid = opaque_tid();
         if (suspended && tid == 0) {
             B.fire[s] = make_float4(fs.dt, fs.damping, (float)fs.lastNeg, 0.f);
             B.nsteps[s] = step;
@@ -744,7 +759,8 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                 B.aforce[I.v0 + v] = make_float4(fo.x, fo.y, fo.z, 0.f);
             }
         }
-        if (B.systime && tid == 0 && P.chunk == 0) B.systime[2 * s + 1] = (long long)wall_clock64();
+        }
+        if (B.systime && threadIdx.x == 0 && P.chunk == 0) B.systime[2 * s + 1] = (long long)wall_clock64();
         __syncthreads();
     }
 }

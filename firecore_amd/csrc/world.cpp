@@ -573,7 +573,6 @@ fcd::BatchDev World::batch_dev() {
     B.bbox = d_bboxes.p;
     B.sysflags = d_sysflags.p;
     B.gridcache = d_gridcache.p;
-    B.gridcache_stride = ntotA;
     B.pbcshifts = d_pbcshifts.p;
     B.neighCell = d_neighCell.p;
     B.snap = (snap_on && d_snap.p) ? d_snap.p : nullptr;
@@ -599,6 +598,8 @@ fcd::RunParams World::run_params(double Fconv, int nstep_max) {
     P.grid.isx = (float)(1.0 / grid.step[0]);
     P.grid.isy = (float)(1.0 / grid.step[1]);
     P.grid.isz = (float)(1.0 / grid.step[2]);
+    P.grid.rnx = 1.f / (float)std::max(grid.nx, 1);
+    P.grid.rny = 1.f / (float)std::max(grid.ny, 1);
     P.fire = fp;
     P.Fconv2 = (float)(Fconv * Fconv);
     P.conv_mode = conv_mode;
@@ -875,7 +876,6 @@ int World::relax_noalloc(int nstep_max, double Fconv, bool restore_start) {
     fcd::BatchDev B = batch_dev();
     B.systime = nullptr;
     B.gridcache = reinterpret_cast<float4*>(base + off_cache);
-    B.gridcache_stride = ntotA;
     fc_launch_zero_f4(stream, d_stall.p, nSys);  // fallback flags of this relaxation only
     fcd::RunParams P = run_params(Fconv, nstep_max);
     hipEvent_t fork = noalloc_events[0];
