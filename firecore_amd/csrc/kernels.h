@@ -73,6 +73,7 @@ struct BatchDev {
     // 0, snap_every, 2*snap_every, ... into snap[k * ntotV + v0 + v], k < nsnap
     float4* snap;
     int snap_every, nsnap, ntotV;
+    int nperiodic;  // periodic molecules in the batch
     // GridFF window cache of the persistent kernel: 16 float4 per atom; the n <= 64
     // atoms of a wave, starting at atom a of the batch, own the run
     // gridcache[16a .. 16(a+n)), row r of the wave's atom l at 16a + r*n + l

@@ -574,6 +574,7 @@ fcd::BatchDev World::batch_dev() {
     B.sysflags = d_sysflags.p;
     B.gridcache = d_gridcache.p;
     B.pbcshifts = d_pbcshifts.p;
+    B.nperiodic = n_periodic;
     B.neighCell = d_neighCell.p;
     B.snap = (snap_on && d_snap.p) ? d_snap.p : nullptr;
     B.snap_every = std::max(snap_every, 1);
