@@ -217,80 +217,104 @@ __global__ void __launch_bounds__(256) k_train_loss_grad(BatchDev B, RunParams P
 }
 
 // ---------------------------------------------------------------- 6. backward
-// dW (64 x KIN) += dZ^T A over the atoms of one system.  A rows: own
-// activation row (chunks < KS) or the bonded-neighbour sum (chunks >= KS).
+// The backward kernel is a workgroup of 8 waves per system, two resident per CU (LDS), and
+// is bound by the latency of its LDS gathers: 512 systems of 16..256 atoms are one
+// resident set, so it takes as long as its largest system.  Hence everything a wave can
+// use twice is read once: a wave owns 16 input columns and all 64 outputs of a weight
+// gradient (the neighbour sums of the input rows are formed once, not per output tile),
+// and 16 output columns of an input gradient with their weights in registers; neighbour
+// lists lie in LDS.  131 us for that batch; with four waves per system that formed the
+// neighbour sums for every output tile and added the biases in one chain, 357 us.
+constexpr int BWD_BLOCK = 512, BWD_NW = BWD_BLOCK / 64;
+
+// dW (64 x KIN) = dZ^T A and db = dZ^T 1 over the atoms of one system.  A rows: own
+// activation row (chunks < KS) or the bonded-neighbour sum (chunks >= KS).  KIN = 128:
+// wave w takes input columns 16w.. and all outputs; KIN = 16: wave w < 4 takes outputs
+// 16w... The bias of outputs 16w.. is wave w's, a product with ones.
 template <int KIN>
-__device__ __forceinline__ void bwd_weight_grad(const unsigned short* dZ, const unsigned short* hin, const int4* nb,
-                                                int n, float* gW) {
+__device__ __forceinline__ void bwd_weight_grad(const unsigned short* dZ, const unsigned short* hin, const short4* nb,
+                                                int n, float* gW, float* gb) {
     constexpr int KS = (KIN == 16) ? 1 : 4;
-    constexpr int NKB = KIN / 16;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    constexpr int NO = (KIN == 16) ? 1 : 4;  // output tiles of a wave
+    static_assert(KIN == 16 || KIN / 16 == BWD_NW, "a wave per 16 input columns");
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (KIN == 16 && wid >= 4) return;
     const int nrb = (n + 15) >> 4;
-    // 4 x NKB output tiles over 4 waves
-    for (int t = wid; t < 4 * NKB; t += 4) {
-        const int ob = t / NKB, kb = t % NKB;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int kc = 0; kc < nrb; kc++) {
-            bf16x4 a, b;
-            const int o = ob * 16 + (lane & 15);
-            const int col = (kb % KS) * 16 + (lane & 15);
+    const int kb = KIN == 16 ? 0 : wid;
+    const int ob0 = KIN == 16 ? wid : 0;
+    const int col = (kb % KS) * 16 + (lane & 15);
+    const bf16x4 ones = {(short)0x3F80, (short)0x3F80, (short)0x3F80, (short)0x3F80};
+    f32x4 acc[NO], accb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < NO; q++) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int kc = 0; kc < nrb; kc++) {
+        bf16x4 b;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int atom = kc * 16 + 4 * (lane >> 4) + i;
+            unsigned short bv = 0;
+            if (atom < n) {
+                if (kb < KS) {
+                    bv = hin[atom * MLP_HS + col];
+                } else {
+                    const int4 n4 = nb_row(nb, atom);
+                    const int ns[4] = {n4.x, n4.y, n4.z, n4.w};
+                    float sacc = 0.f;
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        if (ns[q] >= 0) sacc += bf2f(hin[ns[q] * MLP_HS + col]);
+                    bv = f2bf(sacc);
+                }
+            }
+            b[i] = (short)bv;
+        }
+#pragma unroll
+        for (int q = 0; q < NO; q++) {
+            bf16x4 a;
+            const int o = (ob0 + q) * 16 + (lane & 15);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int atom = kc * 16 + 4 * (lane >> 4) + i;
                 a[i] = (short)((atom < n) ? dZ[atom * MLP_HS + o] : 0);
-                unsigned short bv = 0;
-                if (atom < n) {
-                    if (kb < KS) {
-                        bv = hin[atom * MLP_HS + col];
-                    } else {
-                        const int4 n4 = nb[atom];
-                        const int ns[4] = {n4.x, n4.y, n4.z, n4.w};
-                        float sacc = 0.f;
-#pragma unroll
-                        for (int q = 0; q < 4; q++)
-                            if (ns[q] >= 0) sacc += bf2f(hin[ns[q] * MLP_HS + col]);
-                        bv = f2bf(sacc);
-                    }
-                }
-                b[i] = (short)bv;
             }
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+            acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[q], 0, 0, 0);
+            if (ob0 + q == wid) accb = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, ones, accb, 0, 0, 0);
         }
-        // D[o][k]: lane holds rows 4*(lane/16)+i of column lane%16
+    }
+    // D[o][k]: lane holds rows 4*(lane/16)+i of column lane%16
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int o = ob * 16 + 4 * (lane >> 4) + i;
-            const int k = kb * 16 + (lane & 15);
-            gW[o * KIN + k] = acc[i];
-        }
+    for (int i = 0; i < 4; i++) {
+        const int o = 4 * (lane >> 4) + i;
+#pragma unroll
+        for (int q = 0; q < NO; q++) gW[((ob0 + q) * 16 + o) * KIN + kb * 16 + (lane & 15)] = acc[q][i];
+        if (wid < 4 && (lane & 15) == 0) gb[wid * 16 + o] = accb[i];
     }
 }
 
 // dh (n x 64) = [dZ_i ; sum_nb dZ_j] [W_self^T ; W_nb^T]^T, i.e. the gradient
 // through a 128-input layer back to its 64 inputs (self and neighbour sums
-// share the input rows).  Result tiles in acc (at most 16 per wave).
-__device__ __forceinline__ void bwd_input_grad(const unsigned short* dZ, const int4* nb, const unsigned short* W,
+// share the input rows).  Wave w: columns 16 (w%4).., row blocks w/4 + 2q (acc[q]).
+__device__ __forceinline__ void bwd_input_grad(const unsigned short* dZ, const short4* nb, const unsigned short* W,
                                                int n, f32x4* acc) {
-    constexpr int NW = 4;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nrb = (n + 15) >> 4;
+    const int cb = wid & 3;
+    bf16x4 b[8];
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
+    for (int kc = 0; kc < 8; kc++) {
+        const int col = cb * 16 + (lane & 15) + ((kc >= 4) ? 64 : 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) b[kc][i] = (short)W[((kc & 3) * 16 + 4 * (lane >> 4) + i) * 128 + col];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
         acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const int t = wid + q * NW;
-        if (t < nrb * 4) {
-            const int rb = t >> 2, cb = t & 3;
+        const int rb = (wid >> 2) + 2 * q;
+        if (rb < nrb) {
 #pragma unroll
             for (int kc = 0; kc < 8; kc++) {
                 const bf16x4 a = mlp_a_frag<4>(dZ, nb, n, rb, kc, lane);
-                bf16x4 b;
-                const int col = cb * 16 + (lane & 15) + ((kc >= 4) ? 64 : 0);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int o = (kc & 3) * 16 + 4 * (lane >> 4) + i;
-                    b[i] = (short)W[o * 128 + col];
-                }
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[q], 0, 0, 0);
+                acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[kc], acc[q], 0, 0, 0);
             }
         }
     }
@@ -298,15 +322,13 @@ __device__ __forceinline__ void bwd_input_grad(const unsigned short* dZ, const i
 
 // dz = dh * silu'(z) written as bf16 rows into dZ (after the caller's barrier)
 __device__ __forceinline__ void bwd_store_dz(unsigned short* dZ, const float* z, int n, const f32x4* acc) {
-    constexpr int NW = 4;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int nrb = (n + 15) >> 4;
+    const int col = (wid & 3) * 16 + (lane & 15);
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-        const int t = wid + q * NW;
-        if (t < nrb * 4) {
-            const int rb = t >> 2, cb = t & 3;
-            const int col = cb * 16 + (lane & 15);
+    for (int q = 0; q < 8; q++) {
+        const int rb = (wid >> 2) + 2 * q;
+        if (rb < nrb) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = rb * 16 + 4 * (lane >> 4) + i;
@@ -320,25 +342,17 @@ __device__ __forceinline__ void bwd_store_dz(unsigned short* dZ, const float* z,
     }
 }
 
-__device__ __forceinline__ void bwd_bias_grad(const unsigned short* dZ, int n, float* gb) {
-    for (int k = threadIdx.x; k < MLP_NH; k += blockDim.x) {
-        float s = 0.f;
-        for (int i = 0; i < n; i++) s += bf2f(dZ[i * MLP_HS + k]);
-        gb[k] = s;
-    }
-}
-
-__global__ void __launch_bounds__(256) k_train_bwd(BatchDev B, RunParams P, TrainBufs T) {
-    constexpr int BLOCK = 256;
-    __shared__ __align__(16) unsigned short s_h[BLOCK * MLP_HS];
-    __shared__ __align__(16) unsigned short s_dz[BLOCK * MLP_HS];
-    __shared__ float s_do[2 * BLOCK];
+__global__ void __launch_bounds__(BWD_BLOCK, 4) k_train_bwd(BatchDev B, RunParams P, TrainBufs T) {
+    constexpr int BLOCK = BWD_BLOCK, ROWS = 256;
+    __shared__ __align__(16) unsigned short s_h[ROWS * MLP_HS];
+    __shared__ __align__(16) unsigned short s_dz[ROWS * MLP_HS];
+    __shared__ float s_do[2 * ROWS];
+    __shared__ short4 s_nb[ROWS];
     const int s = blockIdx.x;
     const SysInfo I = B.info[s];
     const int n = I.natoms;
-    if (n > BLOCK || I.nnode > BLOCK) return;
+    if (n > ROWS || I.nnode > ROWS) return;
     const int tid = threadIdx.x;
-    const int4* nb = B.neighs + I.a0;
     const size_t zo = (size_t)3 * MLP_NH * I.a0;
     const float* z1 = T.z + zo;
     const float* z2 = z1 + n * MLP_NH;
@@ -350,21 +364,29 @@ __global__ void __launch_bounds__(256) k_train_bwd(BatchDev B, RunParams P, Trai
     if (tid < n) {
         s_do[tid * 2] = T.dout[(I.a0 + tid) * 2];
         s_do[tid * 2 + 1] = T.dout[(I.a0 + tid) * 2 + 1];
+        const int4 q = B.neighs[I.a0 + tid];
+        s_nb[tid] = make_short4((short)q.x, (short)q.y, (short)q.z, (short)q.w);
     }
     for (int e = tid; e < n * MLP_NH; e += BLOCK) s_h[(e >> 6) * MLP_HS + (e & 63)] = h3[e];
     __syncthreads();
-    // head: dW4[j][k] = sum_i do_ij h3_ik, db4 = sum_i do_i
-    if (tid < 2 * MLP_NH) {
-        const int j = tid >> 6, k = tid & 63;
+    // head: dW4[j][k] = sum_i do_ij h3_ik over a quarter of the atoms each, db4 = sum_i do_i
+    float* s_part = reinterpret_cast<float*>(s_dz);  // not in use yet
+    {
+        const int j = (tid >> 6) & 1, k = tid & 63;
         float sacc = 0.f;
-        for (int i = 0; i < n; i++) sacc += s_do[i * 2 + j] * bf2f(s_h[i * MLP_HS + k]);
-        G[OFF_W4 + j * MLP_NH + k] = sacc;
+#pragma unroll 4
+        for (int i = tid >> 7; i < n; i += 4) sacc += s_do[i * 2 + j] * bf2f(s_h[i * MLP_HS + k]);
+        s_part[tid] = sacc;
     }
+    __syncthreads();
+    if (tid < 2 * MLP_NH)
+        G[OFF_W4 + tid] = (s_part[tid] + s_part[tid + 128]) + (s_part[tid + 256] + s_part[tid + 384]);
     if (tid < 2) {
         float sacc = 0.f;
         for (int i = 0; i < n; i++) sacc += s_do[i * 2 + tid];
         G[OFF_B4 + tid] = sacc;
     }
+    __syncthreads();
     // dz3 = (do W4) * silu'(z3)
     for (int e = tid; e < n * MLP_NH; e += BLOCK) {
         const int i = e >> 6, k = e & 63;
@@ -374,45 +396,57 @@ __global__ void __launch_bounds__(256) k_train_bwd(BatchDev B, RunParams P, Trai
         s_dz[i * MLP_HS + k] = f2bf(dh * sg * (1.f + zz * (1.f - sg)));
     }
     __syncthreads();
-    bwd_bias_grad(s_dz, n, G + OFF_B3);
     // layer 3: input rows h2
     for (int e = tid; e < n * MLP_NH; e += BLOCK) s_h[(e >> 6) * MLP_HS + (e & 63)] = h2[e];
     __syncthreads();
-    bwd_weight_grad<128>(s_dz, s_h, nb, n, G + OFF_W3);
-    f32x4 acc[16];
-    bwd_input_grad(s_dz, nb, P.mlp.W3, n, acc);
+    bwd_weight_grad<128>(s_dz, s_h, s_nb, n, G + OFF_W3, G + OFF_B3);
+    f32x4 acc[8];
+    bwd_input_grad(s_dz, s_nb, P.mlp.W3, n, acc);
     __syncthreads();
     bwd_store_dz(s_dz, z2, n, acc);
     __syncthreads();
-    bwd_bias_grad(s_dz, n, G + OFF_B2);
     // layer 2: input rows h1
     for (int e = tid; e < n * MLP_NH; e += BLOCK) s_h[(e >> 6) * MLP_HS + (e & 63)] = h1[e];
     __syncthreads();
-    bwd_weight_grad<128>(s_dz, s_h, nb, n, G + OFF_W2);
-    bwd_input_grad(s_dz, nb, P.mlp.W2, n, acc);
+    bwd_weight_grad<128>(s_dz, s_h, s_nb, n, G + OFF_W2, G + OFF_B2);
+    bwd_input_grad(s_dz, s_nb, P.mlp.W2, n, acc);
     __syncthreads();
     bwd_store_dz(s_dz, z1, n, acc);
     __syncthreads();
-    bwd_bias_grad(s_dz, n, G + OFF_B1);
     // layer 1: input rows = features
     for (int e = tid; e < n * MLP_NIN; e += BLOCK)
         s_h[(e >> 4) * MLP_HS + (e & 15)] = T.X[(size_t)I.a0 * MLP_NIN + e];
     __syncthreads();
-    bwd_weight_grad<16>(s_dz, s_h, nb, n, G + OFF_W1);
+    bwd_weight_grad<16>(s_dz, s_h, s_nb, n, G + OFF_W1, G + OFF_B1);
 }
 
 // ---------------------------------------------------------------- 7. reduce, 8. Adam
-__global__ void k_grad_reduce(const float* gpart, int nsys, float* grad, const float* loss, float* loss_out) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+// Mean of the systems' gradients: a workgroup takes 64 parameters, its 16 waves every
+// 16th system (256 B per load), and the 16 partial sums are added pairwise.  A thread per
+// parameter over all systems is 70 workgroups with one load in flight each: 148 us for
+// 512 systems (37 MB), 12 us this way (3.1 TB/s).
+constexpr int RED_WAVES = 16;
+__global__ void __launch_bounds__(64 * RED_WAVES) k_grad_reduce(const float* gpart, int nsys, float* grad,
+                                                                const float* loss, float* loss_out) {
+    __shared__ float s_sum[RED_WAVES][64];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
+    float s = 0.f;
     if (p < NPARAM) {
-        float s = 0.f;
-        for (int k = 0; k < nsys; k++) s += gpart[(size_t)k * NPARAM + p];
-        grad[p] = s / (float)nsys;
+#pragma unroll 4
+        for (int k = wid; k < nsys; k += RED_WAVES) s += gpart[(size_t)k * NPARAM + p];
     }
-    if (p == 0) {
+    s_sum[wid][lane] = s;
+    for (int h = RED_WAVES / 2; h > 0; h >>= 1) {
+        __syncthreads();
+        if (wid < h) s_sum[wid][lane] += s_sum[wid + h][lane];
+    }
+    if (wid == 0 && p < NPARAM) grad[p] = s_sum[0][lane] / (float)nsys;
+    if (blockIdx.x == 0 && wid == 1) {
         double l = 0.0;
-        for (int k = 0; k < nsys; k++) l += loss[k];
-        loss_out[0] = (float)(l / nsys);
+        for (int k = lane; k < nsys; k += 64) l += loss[k];
+        l = wave_sum_d(l);
+        if (lane == 0) loss_out[0] = (float)(l / nsys);
     }
 }
 
@@ -460,13 +494,13 @@ extern "C" hipError_t fc_launch_train_loss_grad(hipStream_t st, const fcd::Batch
 }
 extern "C" hipError_t fc_launch_train_bwd(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P,
                                           const fcd::TrainBufs* T) {
-    hipLaunchKernelGGL(fcd::k_train_bwd, dim3(B->nsys), dim3(256), 0, st, *B, *P, *T);
+    hipLaunchKernelGGL(fcd::k_train_bwd, dim3(B->nsys), dim3(fcd::BWD_BLOCK), 0, st, *B, *P, *T);
     return hipGetLastError();
 }
 extern "C" hipError_t fc_launch_grad_reduce(hipStream_t st, const float* gpart, int nsys, float* grad,
                                             const float* loss, float* loss_out) {
-    hipLaunchKernelGGL(fcd::k_grad_reduce, dim3((fcd::NPARAM + 255) / 256), dim3(256), 0, st, gpart, nsys, grad,
-                       loss, loss_out);
+    hipLaunchKernelGGL(fcd::k_grad_reduce, dim3((fcd::NPARAM + 63) / 64), dim3(64 * fcd::RED_WAVES), 0, st, gpart, nsys,
+                       grad, loss, loss_out);
     return hipGetLastError();
 }
 extern "C" hipError_t fc_launch_adam(hipStream_t st, float* theta, float* m, float* v, const float* grad, float lr,
