@@ -198,33 +198,42 @@ __device__ __forceinline__ bf16x4 mlp_b_frag(const unsigned short* W, int cb, in
 // (row block t/4, column block t%4) of [A] W^T, K = KIN (16: the 16 inputs in
 // columns 0..15; 128: own row + neighbour sum).  At most 16 tiles per wave
 // because rows <= BLOCK.
-template <int BLOCK, int KIN>
-__device__ __forceinline__ void mlp_layer(const unsigned short* h, const int4* nb, const unsigned short* W, int n,
+template <int BLOCK, int KIN, class NB>
+__device__ __forceinline__ void mlp_layer(const unsigned short* h, const NB* nb, const unsigned short* W, int n,
                                          int nrb, f32x4* acc) {
     constexpr int NW = BLOCK / 64;
+    static_assert(NW % 4 == 0, "a wave keeps its column block");
     constexpr int NK = KIN / 16;
     constexpr int KS = (KIN == 16) ? 1 : 4;
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
+    // the wave's weights, read once
+    bf16x8 b8[KIN == 128 ? 4 : 1];
+    bf16x4 b4[KIN == 128 ? 1 : NK];
+    if constexpr (KIN == 128) {
+#pragma unroll
+        for (int kc = 0; kc < 4; kc++) b8[kc] = mlp_b_frag32(W, wid & 3, kc, lane);
+    } else {
+#pragma unroll
+        for (int kc = 0; kc < NK; kc++) b4[kc] = mlp_b_frag<KIN>(W, wid & 3, kc, lane);
+    }
 #pragma unroll
     for (int q = 0; q < 16; q++) {
         acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int t = wid + q * NW;
         if (t < nrb * 4) {
-            const int rb = t >> 2, cb = t & 3;
+            const int rb = t >> 2;
             if constexpr (KIN == 128) {
 #pragma unroll
                 for (int kc = 0; kc < 4; kc++) {
                     const bf16x8 a = mlp_a_frag32(h, nb, n, rb, kc, lane);
-                    const bf16x8 b = mlp_b_frag32(W, cb, kc, lane);
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[q], 0, 0, 0);
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b8[kc], acc[q], 0, 0, 0);
                 }
             } else {
 #pragma unroll
                 for (int kc = 0; kc < NK; kc++) {
                     const bf16x4 a = mlp_a_frag<KS>(h, nb, n, rb, kc, lane);
-                    const bf16x4 b = mlp_b_frag<KIN>(W, cb, kc, lane);
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[q], 0, 0, 0);
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b4[kc], acc[q], 0, 0, 0);
                 }
             }
         }
@@ -264,8 +273,8 @@ __device__ __forceinline__ void mlp_store(unsigned short* h, const float* bias, 
 // return out[i*2 + j] = o_ij for i < n.  z (optional, [3][n][64] FP32) and hs
 // (optional, [3][n][64] bf16 rows h1, h2, h3) receive the pre-activations and
 // activations for the backward pass.  Every thread of the block calls it.
-template <int BLOCK>
-__device__ __forceinline__ void mlp_forward(const MlpDev& M, unsigned short* h, const int4* nb, int n, float* out, float* z,
+template <int BLOCK, class NB>
+__device__ __forceinline__ void mlp_forward(const MlpDev& M, unsigned short* h, const NB* nb, int n, float* out, float* z,
                             unsigned short* hs) {
     const int nrb = (n + 15) >> 4;
     f32x4 acc[16];

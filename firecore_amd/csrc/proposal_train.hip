@@ -54,6 +54,8 @@ __global__ void __launch_bounds__(256) k_train_fwd(BatchDev B, RunParams P, Trai
     __shared__ float4 s_F[BLOCK];
     __shared__ __align__(16) unsigned short s_h[BLOCK * MLP_HS];
     __shared__ float s_out[2 * BLOCK];
+    __shared__ short4 s_nb[BLOCK];
+    __shared__ int s_comp[BLOCK];
     const int s = blockIdx.x;
     const SysInfo I = B.info[s];
     const int N = I.natoms, M = I.nnode;
@@ -61,6 +63,11 @@ __global__ void __launch_bounds__(256) k_train_fwd(BatchDev B, RunParams P, Trai
     const int tid = threadIdx.x;
     for (int v = tid; v < N + M; v += BLOCK) s_pos[v] = T.x0[I.v0 + v];
     if (tid < N) s_F[tid] = T.F0[I.v0 + tid];
+    if (tid < N) {
+        const int4 q = B.neighs[I.a0 + tid];
+        s_nb[tid] = make_short4((short)q.x, (short)q.y, (short)q.z, (short)q.w);
+        s_comp[tid] = B.comp[I.a0 + tid];
+    }
     __syncthreads();
     if (tid < N) {
         unsigned short* hrow = s_h + tid * MLP_HS;
@@ -70,7 +77,7 @@ __global__ void __launch_bounds__(256) k_train_fwd(BatchDev B, RunParams P, Trai
     }
     __syncthreads();
     const size_t zo = (size_t)3 * MLP_NH * I.a0;
-    mlp_forward<BLOCK>(P.mlp, s_h, B.neighs + I.a0, N, s_out, T.z + zo, T.hs + zo);
+    mlp_forward<BLOCK>(P.mlp, s_h, s_nb, N, s_out, T.z + zo, T.hs + zo);
     if (tid < N) {
         T.out[(I.a0 + tid) * 2] = s_out[tid * 2];
         T.out[(I.a0 + tid) * 2 + 1] = s_out[tid * 2 + 1];
@@ -80,7 +87,7 @@ __global__ void __launch_bounds__(256) k_train_fwd(BatchDev B, RunParams P, Trai
         float sum = 0.f;
         int cnt = 0;
         for (int i = 0; i < N; i++)
-            if (B.comp[I.a0 + i] == tid) {
+            if (s_comp[i] == tid) {
                 sum += s_out[i * 2 + 1];
                 cnt++;
             }
@@ -117,6 +124,8 @@ __global__ void __launch_bounds__(256) k_train_loss_grad(BatchDev B, RunParams P
     __shared__ float4 s_F1[BLOCK];
     __shared__ float s_red[NW][PC_MAXC][PC_NSUM + 1];
     __shared__ float s_sum[PC_MAXC][PC_NSUM + 1];
+    __shared__ float s_o1[BLOCK];
+    __shared__ int s_comp[BLOCK];
     const int s = blockIdx.x;
     const SysInfo I = B.info[s];
     const int N = I.natoms, M = I.nnode;
@@ -127,6 +136,8 @@ __global__ void __launch_bounds__(256) k_train_loss_grad(BatchDev B, RunParams P
         s_pos[tid] = T.x0[I.v0 + tid];
         s_F0[tid] = T.F0[I.v0 + tid];
         s_F1[tid] = B.aforce[I.v0 + tid];
+        s_o1[tid] = T.out[(I.a0 + tid) * 2 + 1];
+        s_comp[tid] = B.comp[I.a0 + tid];
     }
     __syncthreads();
     const float scale = -T.eta / (float)N;
@@ -209,7 +220,7 @@ __global__ void __launch_bounds__(256) k_train_loss_grad(BatchDev B, RunParams P
         // mean of o1 over the component, as in k_train_fwd
         float sum = 0.f;
         for (int i = 0; i < N; i++)
-            if (B.comp[I.a0 + i] == c) sum += T.out[(I.a0 + i) * 2 + 1];
+            if (s_comp[i] == c) sum += s_o1[i];
         const float sg = sigmoidf_(sum / ncnt);
         T.dout[(I.a0 + tid) * 2 + 1] = scale * s_sum[c][PC_NSUM] * P.pc_grigid * sg * (1.f - sg) / ncnt;
     }
@@ -521,6 +532,8 @@ __global__ void __launch_bounds__(256) k_mlp_gains(BatchDev B, RunParams P, floa
     __shared__ float4 s_F[BLOCK];
     __shared__ __align__(16) unsigned short s_h[BLOCK * MLP_HS];
     __shared__ float s_out[2 * BLOCK];
+    __shared__ short4 s_nb[BLOCK];
+    __shared__ int s_comp[BLOCK];
     const int s = blockIdx.x;
     if (B.status[s] != ST_RUNNING) return;
     const SysInfo I = B.info[s];
@@ -529,18 +542,23 @@ __global__ void __launch_bounds__(256) k_mlp_gains(BatchDev B, RunParams P, floa
     const int tid = threadIdx.x;
     for (int v = tid; v < N + M; v += BLOCK) s_pos[v] = B.atoms[I.v0 + v];
     if (tid < N) s_F[tid] = B.aforce[I.v0 + tid];
+    if (tid < N) {
+        const int4 q = B.neighs[I.a0 + tid];
+        s_nb[tid] = make_short4((short)q.x, (short)q.y, (short)q.z, (short)q.w);
+        s_comp[tid] = B.comp[I.a0 + tid];
+    }
     __syncthreads();
     if (tid < N)
         mlp_feature_row(P, s_pos, s_pos + N, s_F, B.neighs + I.a0, B.elem + I.a0, M, tid, B.PLQs[I.a0 + tid],
                         s_h + tid * MLP_HS);
     __syncthreads();
-    mlp_forward<BLOCK>(P.mlp, s_h, B.neighs + I.a0, N, s_out, nullptr, nullptr);
+    mlp_forward<BLOCK>(P.mlp, s_h, s_nb, N, s_out, nullptr, nullptr);
     if (tid < M) gnode[I.n0 + tid] = P.pc_gstar * sigmoidf_(s_out[tid * 2]);
     if (tid < PC_MAXC) {
         float sum = 0.f;
         int cnt = 0;
         for (int i = 0; i < N; i++)
-            if (B.comp[I.a0 + i] == tid) {
+            if (s_comp[i] == tid) {
                 sum += s_out[i * 2 + 1];
                 cnt++;
             }
