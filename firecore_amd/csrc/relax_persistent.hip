@@ -854,9 +854,15 @@ extern "C" hipError_t fc_noalloc_scratch(void** ptr) {
     return hipSuccess;
 }
 
-extern "C" int fc_lds_bytes(int nmax, int mmax, int block, int learned, int h2lds, int hb) {
+extern "C" int fc_relax_lds_bytes(int nmax, int mmax, int block, int learned, int h2lds, int hb) {
     fcd::LdsLayout L{nmax, mmax, block / 64, learned, h2lds, hb};
     return L.bytes();
+}
+// The same for a batch without H-bond charges (wmax, the exclusion words of an atom,
+// follows from nmax).
+extern "C" int fc_lds_bytes(int nmax, int mmax, int wmax, int block, int learned, int h2lds) {
+    (void)wmax;
+    return fc_relax_lds_bytes(nmax, mmax, block, learned, h2lds, 0);
 }
 
 // bf16 elements of one workgroup's global activation slot (the second buffer)

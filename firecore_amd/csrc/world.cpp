@@ -22,7 +22,7 @@ extern "C" int fc_hslot_elems(int nmax);
 extern "C" hipError_t fc_noalloc_scratch(void** ptr);
 extern "C" hipError_t fc_launch_zero_int(hipStream_t st, int* a, int n);
 extern "C" hipError_t fc_launch_zero_f4(hipStream_t st, float4* a, int n);
-extern "C" int fc_lds_bytes(int nmax, int mmax, int block, int learned, int h2lds, int hb);
+extern "C" int fc_relax_lds_bytes(int nmax, int mmax, int block, int learned, int h2lds, int hb);
 extern "C" hipError_t fc_launch_split_step(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P,
                                            const int* node_sys, int ntot_nodes, int maxN, int do_move, int step);
 extern "C" hipError_t fc_launch_reset(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P);
@@ -704,12 +704,12 @@ void World::plan_classes(bool upload) {
         // learned gains: the second activation buffer goes to LDS when the class
         // keeps two resident workgroups per CU pair of SIMDs (see plan below)
         C.h2lds = 0;
-        C.lds = (size_t)fc_lds_bytes(std::max(C.nmax, 1), std::max(C.mmax, 1), C.block, pc_mode == 2 ? 1 : 0, 0,
-                                     hb_batch ? 1 : 0);
+        C.lds = (size_t)fc_relax_lds_bytes(std::max(C.nmax, 1), std::max(C.mmax, 1), C.block, pc_mode == 2 ? 1 : 0, 0,
+                                           hb_batch ? 1 : 0);
         if (pc_mode == 2 && h2lds_allowed) {
             const size_t budget = (size_t)160 * 1024 / std::max(1, 8 / (C.block / 64));
-            const size_t with = (size_t)fc_lds_bytes(std::max(C.nmax, 1), std::max(C.mmax, 1), C.block, 1, 1,
-                                                     hb_batch ? 1 : 0);
+            const size_t with = (size_t)fc_relax_lds_bytes(std::max(C.nmax, 1), std::max(C.mmax, 1), C.block, 1, 1,
+                                                           hb_batch ? 1 : 0);
             if (with <= budget) {
                 C.h2lds = 1;
                 C.lds = with;
