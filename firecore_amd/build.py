@@ -2,7 +2,9 @@
 
     python -m firecore_amd.build        # or firecore_amd.build.build()
 """
+import json
 import os
+import re
 import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
@@ -18,6 +20,9 @@ ARCH = "gfx950"
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wno-unused-command-line-argument",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 HIP_FLAGS = ["-x", "hip", "--offload-arch=" + ARCH, "-munsafe-fp-atomics", "-fno-hip-fp32-correctly-rounded-divide-sqrt"]
+# the compiler reports what each kernel uses (registers, scratch, LDS): see check_scratch
+RES_FLAGS = ["-Rpass-analysis=kernel-resource-usage"]
+RESOURCES = os.path.join(OBJ, "resources.json")
 HOST_FLAGS = ["-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include"]
 
 HIP_SOURCES = ["relax_persistent.hip", "split_kernels.hip", "sample_kernels.hip", "proposal_train.hip",
@@ -25,24 +30,62 @@ HIP_SOURCES = ["relax_persistent.hip", "split_kernels.hip", "sample_kernels.hip"
 CPP_SOURCES = ["molgen.cpp", "topology.cpp", "gridff_host.cpp", "builder.cpp", "database.cpp", "world.cpp", "train.cpp", "capi.cpp"]
 
 
+def kernel_resources(remarks):
+    """{kernel: {quantity: value}} of the compiler's resource-usage remarks."""
+    out, cur = {}, None
+    for q, v in re.findall(r"remark: +([A-Z][\w ]*?)(?: \[[^\]]*\])?: (\S+) \[-Rpass-analysis=kernel-resource-usage\]",
+                           remarks):
+        if q == "Function Name":
+            cur = out.setdefault(v, {})
+        elif v.isdigit():
+            cur[q] = int(v)
+    return out
+
+
+def check_scratch(res):
+    """No kernel may use scratch memory.  In a build of the relaxation kernel that spilled, the
+    compiler stored a spilled address at a loop exit before it restored the execution mask: the
+    reload gave garbage and the GPU faulted.  Many instances use all 168 registers that three
+    waves per SIMD leave them, so one more live value is enough."""
+    if not res:
+        raise RuntimeError("the compiler gave no resource-usage remarks: cannot tell whether kernels spill")
+    bad = [k for k, r in res.items() if r["ScratchSize"] or r["VGPRs Spill"]]
+    if bad:
+        raise RuntimeError("kernels with scratch memory (register spills): " + ", ".join(
+            "%s (%d B per lane, %d VGPRs)" % (k, res[k]["ScratchSize"], res[k]["VGPRs Spill"]) for k in bad))
+
+
+def resources():
+    """What the kernels of the last build use."""
+    with open(RESOURCES) as f:
+        return json.load(f)
+
+
 def _compile(src):
     path = os.path.join(CSRC, src)
     obj = os.path.join(OBJ, src + ".o")
     if src.endswith(".hip"):
-        cmd = [HIPCC] + COMMON + HIP_FLAGS + ["-c", path, "-o", obj]
+        cmd = [HIPCC] + COMMON + HIP_FLAGS + RES_FLAGS + ["-c", path, "-o", obj]
     else:
         cmd = [HIPCC] + COMMON + HOST_FLAGS + ["-c", path, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("compile failed: %s\n%s\n%s" % (" ".join(cmd), r.stdout, r.stderr))
-    return obj
+    if not src.endswith(".hip"):
+        return obj, {}
+    res = kernel_resources(r.stderr)
+    check_scratch(res)
+    return obj, res
 
 
 def build(verbose=False):
     os.makedirs(OBJ, exist_ok=True)
     srcs = HIP_SOURCES + CPP_SOURCES
     with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
-        objs = list(ex.map(_compile, srcs))
+        done = list(ex.map(_compile, srcs))
+    objs = [obj for obj, _ in done]
+    with open(RESOURCES, "w") as f:
+        json.dump({k: r for _, res in done for k, r in res.items()}, f, indent=1)
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "-shared", "-fPIC", "--offload-arch=" + ARCH, "-o", tmp] + objs + ["-lpthread"]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -106,14 +106,9 @@ struct Queues {
 };
 
 // minimum resident waves per SIMD the register allocation must allow
-#ifndef FC_WAVES_PER_SIMD
-#define FC_WAVES_PER_SIMD 3
-#endif
-#ifndef FC_WAVES_PER_SIMD_LEARNED
-#define FC_WAVES_PER_SIMD_LEARNED FC_WAVES_PER_SIMD
-#endif
+constexpr int WAVES_PER_SIMD = 3;
 template <int BLOCK, bool HB, int PC>
-__global__ void __launch_bounds__(BLOCK, PC == 2 ? FC_WAVES_PER_SIMD_LEARNED : FC_WAVES_PER_SIMD)
+__global__ void __launch_bounds__(BLOCK, WAVES_PER_SIMD)
 relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                                                                  LdsLayout L) {
     extern __shared__ float4 lds_dyn[];
