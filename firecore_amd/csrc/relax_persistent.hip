@@ -382,7 +382,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     float4* slots = B.gridcache + (size_t)(I.a0 + wu * 64) * 16;
                     const int nslot = min(64, N - wu * 64);
                     if (onGrid) gw.refill(P.grid, lane, plq, slots, nslot);
-                    if (wu < nwAct) {
+                    if (wu < nwAct && (P.bNonBonded || onGrid)) {
                         const int ia = hasAtom ? tid : 0;
                         const float4* pp = s_pos + ia;
                         const float2* pr = s_re + ia;
@@ -427,7 +427,10 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                         a0 = rows(0);
                         a1 = rows(1);
                         unsigned keep = 0;
-                        const int Kn = (Kl & ~3) + 4;  // offsets taken: 0..Kn-1
+                        // offsets taken: 0..Kn-1.  Without non-bonded terms one masked iteration,
+                        // for the window's halves, and no loop at all in vacuum: all offsets masked
+                        // took 68 us a step for 4096 vacuum systems of 16..256 atoms, this 22.
+                        const int Kn = P.bNonBonded ? (Kl & ~3) + 4 : 4;
                         const int kmid = (Kn >> 3) << 2;
                         if (onGrid) gw.fetch(hasAtom ? lane : 0, slots, nslot, 0);
                         else gw.no_fetch();
