@@ -23,6 +23,7 @@
 namespace fcd {
 
 constexpr int PC_MAXC = 4;  // components per system handled by the molecule-level projection
+constexpr int PC_NFIT = 10;  // a component's rigid fit: count, centroid(3), mean force(3), angular rate(3)
 constexpr int PC_NSUM = 16; // reduced sums per component: n, sum r(3), sum F(3), sum r x F(3), sum r r^T(6)
 
 // Solve (I + eps*tr(I)) w = b for a symmetric 3x3 I = (xx, yy, zz, xy, xz, yz).
@@ -213,7 +214,7 @@ __device__ __forceinline__ void precondition(const RunParams& P, const float4* s
     }
     __syncthreads();
     // one thread per component: block totals and the rigid-body fit, kept in
-    // s_csum[c*16]: count, centroid (1..3), mean force t (4..6), angular rate w (7..9)
+    // s_csum[c*PC_NFIT]: count, centroid (1..3), mean force t (4..6), angular rate w (7..9)
     if (tid < nc) {
         float S[PC_NSUM];
 #pragma unroll
@@ -225,7 +226,7 @@ __device__ __forceinline__ void precondition(const RunParams& P, const float4* s
         }
         V3 cen, t, w;
         comp_rigid(S, cen, t, w);
-        float* o = s_csum + tid * PC_NSUM;
+        float* o = s_csum + tid * PC_NFIT;
         o[0] = S[0];
         o[1] = cen.x;
         o[2] = cen.y;
@@ -273,7 +274,7 @@ __device__ __forceinline__ void precondition(const RunParams& P, const float4* s
             if (b4[k] < 0) break;
             f += xyz(s_fng[b4[k]]);
         }
-        const float* o = s_csum + myc * PC_NSUM;
+        const float* o = s_csum + myc * PC_NFIT;
         const V3 cen = mk(o[1], o[2], o[3]), t = mk(o[4], o[5], o[6]), w = mk(o[7], o[8], o[9]);
         const float gc = learned ? s_gain[M + myc] : P.pc_grigid;
         f += (t + cross(w, r - cen)) * gc;

@@ -38,54 +38,65 @@ __device__ __forceinline__ int4 unpack4(uint2 p) {
 }
 
 // LDS layout (bytes), computed identically on the host (world.cpp).
-//   pos   float4[prow+mmax]     (x, y, z, Q) of the atoms as periodic rows: row r
+//   pos   float4[prow]          (x, y, z, Q) of the atoms as periodic rows: row r
 //                              holds atom r mod N, so the partners of an atom at
-//                              offsets 0..N/2 follow it without a wrap; then the
-//                              pi-vectors, from row prow
-//   re    float2[prow]          (R0, sqrt(E0)) in the same rows
-//   hb    float[prow]           H of the same rows (batches with H-bond charges)
-//   fnb   float4[nmax]          non-bonded + grid force accumulated by atom i's thread
+//                              offsets 0..N/2 follow it without a wrap
+//   pi    float4[mmax]          pi-vectors
+//   fnb   float4[nmax]          bonded self force of node i; with gains (precond.h) the
+//                              exact force of atom i afterwards
+//   re    float2[prow]          (R0, sqrt(E0)) in the rows of pos
+//   hb    float[prow]           H in the same rows (batches with H-bond charges)
 //   facc  float4[nwave*frow]    per-wave reaction forces of the half-ring schedule:
 //                              entry e of wave w's row is the reaction on atom
 //                              (64w+e) mod N
-//   fself float4[2*mmax]        bonded self forces of nodes and pi-vectors
+//   fself float4[mmax]          bonded self forces of the pi-vectors
 //   fng   float4[8*mmax]        recoils (sigma rows, then pi rows)
 //   mask  uint[wmax*nmax]       rotated exclusion rows, [word][atom]: the whole words
 //                              below the one of the last offset, which each
 //                              thread keeps in a register
 //   learned gains only:
-//   gain  float[mmax+PC_MAXC]   gains of the stars and the components
-//   h     bf16 rows            network activations (one of the two buffers),
-//                              aliased onto facc..mask, which is padded to fit
+//   h     bf16 rows            network activations (one of the two buffers), over
+//                              re..mask, which the next step needs again or rewrites
+//   nb    short4[nmax]          bonded neighbours during the network evaluation, after h
+//   gain  float[mmax+PC_MAXC]   gains of the stars and the components, after all of these
+//
+// The step is bound by how many waves a CU holds, and LDS is given out in units of
+// 1280 B: a form that exceeds 53760 B at 256 atoms, static part included, runs two
+// workgroups there instead of three.  Rows that only their own thread reads are not kept
+// twice, which pays for the periodic rows: no size and form needs more than with plain
+// rows and wrapped indices, and 256 atoms with up to 128 nodes run three workgroups in
+// every form; 768 of them with H-bond charges and constant gains take 45 us a step, with
+// two workgroups per CU 54.
 struct LdsLayout {
     int nmax, mmax, nwave, learned, h2lds, hb;
     __host__ __device__ static int r16(int b) { return (b + 15) & ~15; }
-    // rows the pair loop reads: offsets 0..N/2, rounded up to whole iterations, and
-    // the next iteration's first rows read ahead
-    __host__ __device__ static int prow_of(int n) { return n + (n >> 1) + 8; }
+    // rows of the pairs the loop computes: offsets 0..N/2 rounded up to whole iterations.
+    // The rows it reads ahead in the last iteration, and does not use, are two more: they
+    // lie in the next array.
+    __host__ __device__ static int prow_of(int n) { return n + (n >> 1) + 3; }
     __host__ __device__ int prow() const { return prow_of(nmax); }
     __host__ __device__ int wmax() const { return nmax >> 6; }
     __host__ __device__ int off_pos() const { return 0; }
-    __host__ __device__ int off_re() const { return off_pos() + (prow() + mmax) * 16; }
+    __host__ __device__ int off_pi() const { return off_pos() + prow() * 16; }
+    __host__ __device__ int off_fnb() const { return off_pi() + mmax * 16; }
+    __host__ __device__ int off_re() const { return off_fnb() + nmax * 16; }
     __host__ __device__ int off_hb() const { return off_re() + r16(prow() * 8); }
-    __host__ __device__ int off_fnb() const { return off_hb() + (hb ? r16(prow() * 4) : 0); }
-    __host__ __device__ int off_facc() const { return off_fnb() + nmax * 16; }
+    __host__ __device__ int off_facc() const { return off_hb() + (hb ? r16(prow() * 4) : 0); }
     // entries of a wave's reaction row: lane l's partner at offset k lands at l+k
-    __host__ __device__ int frow() const { return 64 + (nmax >> 1) + 4; }
+    __host__ __device__ int frow() const { return 64 + (nmax >> 1); }
     __host__ __device__ int off_fself() const { return off_facc() + nwave * frow() * 16; }
-    __host__ __device__ int off_fng() const { return off_fself() + 2 * mmax * 16; }
+    __host__ __device__ int off_fng() const { return off_fself() + mmax * 16; }
     __host__ __device__ int off_mask() const { return off_fng() + 8 * mmax * 16; }
     __host__ __device__ int end_base() const { return off_mask() + nmax * wmax() * 4; }
     __host__ __device__ int hbytes() const { return r16(nmax * MLP_HS * 2); }
+    __host__ __device__ int off_h() const { return off_re(); }
+    __host__ __device__ int off_nb() const { return off_h() + hbytes(); }
     __host__ __device__ int off_gain() const {
-        const int e = end_base();
-        return r16((learned && off_facc() + hbytes() > e) ? off_facc() + hbytes() : e);
+        const int e = end_base(), n = off_nb() + nmax * 8;
+        return r16((learned && n > e) ? n : e);
     }
-    __host__ __device__ int off_hx() const { return off_gain() + r16((mmax + PC_MAXC) * 4); }
-    // first activation buffer: in LDS over facc..mask, which is free during the
-    // network evaluation (the exclusion rows are staged again after it) and is
-    // padded to hold it (off_gain)
-    __host__ __device__ int off_h2() const { return off_hx(); }
+    // the second activation buffer, where it is kept in LDS
+    __host__ __device__ int off_h2() const { return off_gain() + r16((mmax + PC_MAXC) * 4); }
     __host__ __device__ int bytes() const {
         if (!learned) return end_base();
         return off_h2() + (h2lds ? hbytes() : 0);
@@ -114,7 +125,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
     extern __shared__ float4 lds_dyn[];
     char* lds = reinterpret_cast<char*>(lds_dyn);
     float4* s_pos = reinterpret_cast<float4*>(lds + L.off_pos());
-    float4* s_pi = s_pos + L.prow();
+    float4* s_pi = reinterpret_cast<float4*>(lds + L.off_pi());
     float2* s_re = reinterpret_cast<float2*>(lds + L.off_re());
     float* s_hb = reinterpret_cast<float*>(lds + L.off_hb());
     float4* s_fnb = reinterpret_cast<float4*>(lds + L.off_fnb());
@@ -125,7 +136,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
     float* s_gain = reinterpret_cast<float*>(lds + L.off_gain());
     // activation buffers of the in-kernel network: LDS where the layout allows,
     // else the two halves of this workgroup's global slot
-    unsigned short* s_h = reinterpret_cast<unsigned short*>(lds + L.off_facc());
+    unsigned short* s_h = reinterpret_cast<unsigned short*>(lds + L.off_h());
     unsigned short* g_h = L.h2lds ? reinterpret_cast<unsigned short*>(lds + L.off_h2())
                                   : (Q.hslot ? Q.hslot + (size_t)blockIdx.x * (L.hbytes() / 2) : nullptr);
     const bool learned = PC >= 2 && L.learned && P.pc_mode == 2;
@@ -134,9 +145,9 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
     __shared__ float s_red[4][2 * NW];
     __shared__ double s_redd[NW];
     __shared__ int s_q;
-    // preconditioner: per-wave partial sums and per-component totals (PC_NSUM values each)
+    // preconditioner: per-wave partial sums and the fit of each component
     __shared__ float s_cred[PC ? NW : 1][PC ? PC_MAXC : 1][PC_NSUM];
-    __shared__ float s_csum[PC ? PC_MAXC : 1][PC_NSUM];
+    __shared__ float s_csum[PC ? PC_MAXC : 1][PC_NFIT];
     __shared__ float s_smax[NW];
     __shared__ float s_st_best;       // FIRE fallback of the learned form (below)
     __shared__ int s_st_cnt, s_st_plain;
@@ -376,8 +387,8 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                                     [&](int k, V3 g) { put(4 * M + tid * 4 + k, g); }, fbs, fa, fpi);
 #pragma unroll
                         for (int k = 0; k < 4; k++) put(tid * 4 + k, fbs[k]);
-                        s_fself[tid] = make_float4(fa.x, fa.y, fa.z, 0.f);
-                        s_fself[M + tid] = make_float4(fpi.x, fpi.y, fpi.z, 0.f);
+                        s_fnb[tid] = make_float4(fa.x, fa.y, fa.z, 0.f);
+                        s_fself[tid] = make_float4(fpi.x, fpi.y, fpi.z, 0.f);
                     }
                     float4* slots = B.gridcache + (size_t)(I.a0 + wu * 64) * 16;
                     const int nslot = min(64, N - wu * 64);
@@ -483,7 +494,8 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                             fout += 64;
                         }
                         if (onGrid) gw.add(1);
-                        s_facc[wu * L.frow() + Kn - 1 + lane] = make_float4(acc.x, acc.y, acc.z, 0.f);
+                        if (Kn - 1 + lane < nrow)
+                            s_facc[wu * L.frow() + Kn - 1 + lane] = make_float4(acc.x, acc.y, acc.z, 0.f);
                     }
                     if (hasAtom) {
                         const int i = tid;
@@ -502,7 +514,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                         }
                     }
                     if (onGrid) gw.finish(P.grid, f);
-                    if (hasAtom) s_fnb[tid] = make_float4(f.x, f.y, f.z, 0.f);
+                    const V3 fnb = f;  // non-bonded and grid force on atom tid
                     __syncthreads();
 
                     // ================= B: assemble + reductions
@@ -512,9 +524,9 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                         fv[r] = zero3();
                         if (v < V) {
                             V3 f = zero3();
-                            const bool isPi = v >= N;
+                            const bool isPi = r > 0 || v >= N;  // N <= BLOCK
                             if (!isPi) {
-                                f = xyz(s_fnb[v]);
+                                f = fnb;
                                 if (P.bNonBonded && N >= 2)
                                     for (int w = 0; w < nwAct; w++) {  // atom v: entries (v-64w) mod N + multiples of N
                                         int e = v - 64 * w;            // > -N: an active wave's first atom is below N
@@ -522,14 +534,14 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                                         const float4* row = s_facc + w * L.frow();
                                         for (; e < nrow; e += N) f += xyz(row[e]);
                                     }
-                                if (v < M) f += xyz(s_fself[v]);
+                                if (v < M) f += xyz(s_fnb[v]);
                                 if (sflags) {  // restraints and walls are part of the exact force
                                     const V3 p = xyz(s_pos[v]);
                                     if (sflags & 1) f += restraint_force(p, B.constr[I.a0 + v], B.constrK[I.a0 + v]);
                                     if (sflags & 2) f += wall_force(p, B.bbox[3 * s], B.bbox[3 * s + 1], B.bbox[3 * s + 2]);
                                 }
                             } else {
-                                f = xyz(s_fself[M + (v - N)]);
+                                f = xyz(s_fself[v - N]);
                             }
                             const int4 b = unpack4(bkp[r]);
                             const int b4[4] = {b.x, b.y, b.z, b.w};
@@ -698,7 +710,8 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                         if (isPi) {
                             s_pi[v - N] = make_float4(p.x, p.y, p.z, 0.f);
                         } else {
-                            // the atom's periodic rows (two, more below 17 atoms); Q stays
+                            // the atom's periodic rows (a second one below N/2 + 3, a third
+                            // only in molecules of less than 5 atoms); Q stays
                             const f32x3 t = {p.x, p.y, p.z};
                             *reinterpret_cast<f32x3*>(s_pos + v) = t;
                             for (int q = v + N; q < PR; q += N) *reinterpret_cast<f32x3*>(s_pos + q) = t;
@@ -721,10 +734,10 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
             }
             __syncthreads();
             propose_gains<BLOCK>(P, B.neighs + I.a0, B.elem + I.a0, s_pos, s_pi, s_fnb,
-                                 reinterpret_cast<short4*>(s_re), s_h, g_h, s_gain, &s_cred[0][0][0], N, M, nc, hasAtom ? B.comp[I.a0 + tid] : 0,
+                                 reinterpret_cast<short4*>(lds + L.off_nb()), s_h, g_h, s_gain, &s_cred[0][0][0], N, M, nc, hasAtom ? B.comp[I.a0 + tid] : 0,
                                  hasAtom ? B.PLQs[I.a0 + tid] : make_float4(0, 0, 0, 0));
-            stage_mask();  // the exclusion rows were overwritten by the activations,
-            stage_re();    // the pair parameters by the neighbour lists
+            stage_mask();  // the exclusion rows and the pair parameters were overwritten
+            stage_re();    // by the activations
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 const int v = tid + r * BLOCK;
@@ -855,6 +868,14 @@ extern "C" hipError_t fc_noalloc_scratch(void** ptr) {
 extern "C" int fc_relax_lds_bytes(int nmax, int mmax, int block, int learned, int h2lds, int hb) {
     fcd::LdsLayout L{nmax, mmax, block / 64, learned, h2lds, hb};
     return L.bytes();
+}
+// Where its arrays begin, in the order of the layout's list above, then the second
+// activation buffer and the end.
+extern "C" void fc_relax_lds_offsets(int nmax, int mmax, int block, int learned, int h2lds, int hb, int* out) {
+    fcd::LdsLayout L{nmax, mmax, block / 64, learned, h2lds, hb};
+    const int o[] = {L.off_pos(), L.off_pi(), L.off_fnb(), L.off_re(), L.off_hb(), L.off_facc(), L.off_fself(),
+                     L.off_fng(), L.off_mask(), L.off_h(), L.off_nb(), L.off_gain(), L.off_h2(), L.bytes()};
+    for (size_t k = 0; k < sizeof(o) / sizeof(o[0]); k++) out[k] = o[k];
 }
 // The same for a batch without H-bond charges (wmax, the exclusion words of an atom,
 // follows from nmax).

@@ -539,7 +539,7 @@ __global__ void __launch_bounds__(256) k_precond(BatchDev B, RunParams P, float4
     __shared__ float4 s_fself[BLOCK];
     __shared__ float4 s_fng[4 * BLOCK];
     __shared__ float s_cred[NW][PC_MAXC][PC_NSUM];
-    __shared__ float s_csum[PC_MAXC][PC_NSUM];
+    __shared__ float s_csum[PC_MAXC][PC_NFIT];
     __shared__ float s_gain[BLOCK + PC_MAXC];
     const int s = blockIdx.x;
     const SysInfo I = B.info[s];
