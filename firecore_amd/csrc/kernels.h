@@ -73,7 +73,6 @@ struct BatchDev {
     // 0, snap_every, 2*snap_every, ... into snap[k * ntotV + v0 + v], k < nsnap
     float4* snap;
     int snap_every, nsnap, ntotV;
-    int nperiodic;  // periodic molecules in the batch
     // GridFF window cache of the persistent kernel: 16 float4 per atom; the n <= 64
     // atoms of a wave, starting at atom a of the batch, own the run
     // gridcache[16a .. 16(a+n)), row r of the wave's atom l at 16a + r*n + l
@@ -105,6 +104,15 @@ struct BatchDev {
     int4* xstate;
     double* minE;
     float4* minpos;
+};
+
+// Which systems the non-bonded kernels of a split step take how: those of lane_sys[0 ..
+// lane_n) (null: systems 0 .. lane_n) with a wave per atom, the largest of lane_maxN atoms;
+// the vacuum molecules of the batch with a thread per atom, the largest of tile_maxN
+// (0: none of them).
+struct NonbondPlan {
+    const int* lane_sys;
+    int lane_n, lane_maxN, tile_maxN;
 };
 
 // Parameters of the proposal network (BF16 dense layers, FP32 head).

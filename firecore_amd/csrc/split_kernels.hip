@@ -10,11 +10,12 @@
 
 namespace fcd {
 
-// The (atom j, image s) pairs of a lane: every 64th of the list that has the n images
+// The (atom j, image s) pairs of a lane: every L-th of the list that has the n images
 // of an atom next to each other.
+template <int L>
 struct LanePairs {
     int j, s, n, dj, ds;
-    __device__ LanePairs(int lane, int n_) : j(lane / n_), s(lane % n_), n(n_), dj(64 / n_), ds(64 % n_) {}
+    __device__ LanePairs(int lane, int n_) : j(lane / n_), s(lane % n_), n(n_), dj(L / n_), ds(L % n_) {}
     __device__ void next() {
         s += ds;
         j += dj + (s >= n ? 1 : 0);
@@ -38,7 +39,7 @@ __device__ void nb_pbc_atom(const BatchDev& B, const SysInfo& I, int i, V3 pi, f
     const float4* sh = B.pbcshifts + I.sh0;
     const int4 ng = B.neighs[I.a0 + i];
     const int4 nc = B.neighCell[I.a0 + i];
-    LanePairs t(lane, I.npbc);
+    LanePairs<64> t(lane, I.npbc);
 #pragma unroll 2
     for (; t.j < I.natoms; t.next()) {
         const int j = t.j, s = t.s;
@@ -75,18 +76,15 @@ __device__ void nb_pbc_atom(const BatchDev& B, const SysInfo& I, int i, V3 pi, f
 // (REQs mixed by combineREQ: R0 sum, E0 and charge products) at every image
 // shift, dp = pi - pj - shift, r = |dp|, e = exp(K (r - R0)) with K =
 // -alphaMorse; E = E0 e (e - 2) + k q q / r and the force on i is
-// -dp (2 K E0 e (e - 1) / r - k q q / r^3).  Adds this lane's share of the
-// force to f, returns its share of E.
+// -dp (2 K E0 e (e - 1) / r - k q q / r^3).  Adds the force of every L-th
+// term, from term `lane`, to f and returns their E.
+template <int L>
 __device__ float surf_atoms_force(const RunParams& P, V3 pi, float4 ri, int lane, V3& f) {
     float E = 0.f;
     const float K = P.surf_K;
-    LanePairs t(lane, P.nsurf_pbc);
-#pragma unroll 2
-    for (; t.j < P.nsurf; t.next()) {
-        const float4 a = P.surf_pos[t.j];
-        const float4 q = P.surf_REQ[t.j];
+    auto term = [&](float4 a, float4 q, int shift) {
         const float r0 = q.x + ri.x, e0 = q.y * ri.y, kqq = COULOMB_K * q.z * ri.z;
-        const V3 dp = mk(pi.x - a.x, pi.y - a.y, pi.z - a.z) + xyz(P.surf_shifts[t.s]);
+        const V3 dp = mk(pi.x - a.x, pi.y - a.y, pi.z - a.z) + xyz(P.surf_shifts[shift]);
         const float r2 = dot(dp, dp);
         const float ir = __builtin_amdgcn_rsqf(r2);
         const float r = r2 * ir;
@@ -96,22 +94,143 @@ __device__ float surf_atoms_force(const RunParams& P, V3 pi, float4 ri, int lane
         E += Ae * (e - 2.f) + eel;
         const float fr = 2.f * K * Ae * (e - 1.f) * ir - eel * ir * ir;
         f -= dp * fr;
+    };
+    if constexpr (L == 1) {
+        for (int j = 0; j < P.nsurf; j++) {
+            const float4 a = P.surf_pos[j], q = P.surf_REQ[j];
+            for (int s = 0; s < P.nsurf_pbc; s++) term(a, q, s);
+        }
+    } else {
+        LanePairs<L> t(lane, P.nsurf_pbc);
+#pragma unroll 2
+        for (; t.j < P.nsurf; t.next()) term(P.surf_pos[t.j], P.surf_REQ[t.j], t.s);
     }
     return E;
 }
 
 // ---------------------------------------------------------------------------
-// Non-bonded (+GridFF) force per atom.  grid = (ceil(maxN/64), nsys), 64 threads.
-// aforce[v0+i] = (f, 0.5*E_nb + E_grid)   (assignment, like the reference NB kernel)
-__global__ void __launch_bounds__(64) k_nonbond_grid(BatchDev B, RunParams P) {
+// Lane (a, b, c) = (lane >> 4, lane >> 2 & 3, lane & 3)'s share of grid_sample: the one
+// coefficient of the 4x4x4 window that is its own (a wave per atom would otherwise gather
+// all 64 in every lane).
+__device__ float grid_sample_lane(const GridDev& g, V3 p, V3 plq, int lane, V3& f) {
+    const float ux = (p.x - g.p0x) * g.isx;
+    const float uy = (p.y - g.p0y) * g.isy;
+    const float uz = (p.z - g.p0z) * g.isz;
+    int ix = (int)ux, iy = (int)uy, iz = (int)uz;
+    if (ux < 0.f) ix--;
+    if (uy < 0.f) iy--;
+    const float tx = ux - ix, ty = uy - iy, tz = uz - iz;
+    iz = min(max(iz, 3), g.nz - 5) + (lane & 3) - 1;
+    ix = imod(ix - 1, g.nx) + (lane >> 4);
+    iy = imod(iy - 1, g.ny) + ((lane >> 2) & 3);
+    if (ix >= g.nx) ix -= g.nx;
+    if (iy >= g.ny) iy -= g.ny;
+    const float4 q = g.coefs[(size_t)(ix * g.ny + iy) * g.nz + iz];
+    // weights in registers: an array indexed by the lane would go to LDS
+    auto pick = [](int k, const float* w) {
+        const float w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
+        const float lo = k & 1 ? w1 : w0, hi = k & 1 ? w3 : w2;
+        return k & 2 ? hi : lo;
+    };
+    const int la = lane >> 4, lb = (lane >> 2) & 3, lc = lane & 3;
+    float wx[4], vx[4], wy[4], vy[4], wz[4], vz[4];
+    bs_basis(tx, wx);
+    bs_dbasis(tx, vx);
+    bs_basis(ty, wy);
+    bs_dbasis(ty, vy);
+    bs_basis(tz, wz);
+    bs_dbasis(tz, vz);
+    const float bx = pick(la, wx), by = pick(lb, wy), bz = pick(lc, wz);
+    const float dx = pick(la, vx), dy = pick(lb, vy), dz = pick(lc, vz);
+    const float c = plq.x * q.x + plq.y * q.y + plq.z * q.z;
+    f.x -= c * bz * by * dx * g.isx;
+    f.y -= c * bz * dy * bx * g.isy;
+    f.z -= c * dz * by * bx * g.isz;
+    return c * bz * by * bx;
+}
+
+// ---------------------------------------------------------------------------
+// Non-bonded (+GridFF) force on atom i of system s by a whole wave: lane l takes every
+// 64th term, partners and images as one index; the 64 partial sums are added by a
+// butterfly.  aforce[v0+i] = f, enb[a0+i] = 0.5*E_nb + E_grid (assignment).
+__device__ void nb_wave_atom(const BatchDev& B, const RunParams& P, int s, int i, int lane) {
+    const SysInfo I = B.info[s];
+    const int N = I.natoms;
+    if (i >= N) return;
+    const V3 pi = xyz(B.atoms[I.v0 + i]);
+    const float4 ri = B.REQs[I.a0 + i];
+    const float kQi = COULOMB_K * ri.z;
+    V3 f = zero3();
+    double e = 0.0;  // FP64 accumulation of the pair energies
+    if (P.bNonBonded && I.npbc > 0) {
+        nb_pbc_atom(B, I, i, pi, ri, lane, f, e);
+    } else if (P.bNonBonded) {
+        const unsigned* ex = B.excl + I.mask0 + i * ((N + 31) >> 5);
+        for (int j = lane; j < N; j += 64) {
+            const V3 d = xyz(B.atoms[I.v0 + j]) - pi;
+            const float4 rj = B.REQs[I.a0 + j];
+            if ((ex[j >> 5] >> (j & 31)) & 1u) continue;  // the atom itself among them
+            float fr, ep;
+            lj_pair<true, true>(d, ri.x + rj.x, ri.y * rj.y, kQi * rj.z, ri.w * rj.w, fr, ep);
+            f -= d * fr;
+            e += (double)ep;
+        }
+        for (int c = lane; c < I.ncorr; c += 64) {
+            const PairCorrDev pc = B.corr[I.corr0 + c];
+            if (pc.i != i) continue;
+            const V3 d = xyz(B.atoms[I.v0 + pc.j]) - pi;
+            const float4 rj = B.REQs[I.a0 + pc.j];
+            float fr, ep;
+            lj_pair<true, true>(d, ri.x + rj.x, ri.y * rj.y, kQi * rj.z, ri.w * rj.w, fr, ep);
+            f -= d * (fr * pc.w);
+            e += (double)ep * pc.w;
+        }
+    }
+    e *= 0.5;
+    if (P.nsurf > 0 && P.nsurf_pbc > 0) e += (double)surf_atoms_force<64>(P, pi, ri, lane, f);
+    if (P.bGridFF) e += (double)grid_sample_lane(P.grid, pi, xyz(B.PLQs[I.a0 + i]), lane, f);
+    f = mk(wave_sum(f.x), wave_sum(f.y), wave_sum(f.z));
+    e = wave_sum_d(e);
+    if (lane != 0) return;
+    B.aforce[I.v0 + i] = make_float4(f.x, f.y, f.z, 0.f);
+    B.enb[I.a0 + i] = e;
+}
+
+// For periodic molecules and small batches over substrate atoms (World::nonbond_plan draws
+// the line): atoms x images are hundreds to thousands of terms with a root, an exponential
+// or a division each, a long chain for one thread.  32 molecules of 40..96 atoms with 9
+// images take 28 us a step, all launches included (241 with a thread per atom), 2048 of
+// them, which fill the card, 279 (372), over the grid 298 (380).
+// grid = (ceil(maxN/4), systems), 256 threads; no barrier, a wave may end on its own.
+__global__ void __launch_bounds__(256) k_nonbond_lanes(BatchDev B, RunParams P, NonbondPlan nb) {
+    const int s = nb.lane_sys ? nb.lane_sys[blockIdx.y] : blockIdx.y;
+    if (B.status[s] != ST_RUNNING) return;
+    nb_wave_atom(B, P, s, blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
+}
+
+// ---------------------------------------------------------------------------
+// Non-bonded (+GridFF) force per atom, like the reference NB kernel: vacuum molecules with
+// a thread per atom and the partners in LDS, in ceil(tile_maxN/64) workgroups of 64 threads
+// each; before them the atoms of the periodic molecules, a wave each.
+__global__ void __launch_bounds__(64) k_nonbond_grid(BatchDev B, RunParams P, NonbondPlan nb) {
     __shared__ float4 s_p[64];
     __shared__ float4 s_r[64];
-    const int s = blockIdx.y;
+    int b = blockIdx.x;
+    if (b < nb.lane_n * nb.lane_maxN) {
+        const int q = b / nb.lane_maxN;
+        const int s = nb.lane_sys[q];
+        if (B.status[s] == ST_RUNNING) nb_wave_atom(B, P, s, b - q * nb.lane_maxN, threadIdx.x);
+        return;
+    }
+    b -= nb.lane_n * nb.lane_maxN;
+    const int tiles = (nb.tile_maxN + 63) >> 6;
+    const int s = b / tiles;
+    const int i0 = (b - s * tiles) * 64;
     const SysInfo I = B.info[s];
     if (B.status[s] != ST_RUNNING) return;
     const int N = I.natoms;
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    if (blockIdx.x * 64 >= N) return;
+    const int i = i0 + threadIdx.x;
+    if (i0 >= N || I.npbc > 0) return;
     const bool act = i < N;
     const int W = (N + 31) >> 5;
     V3 pi = zero3();
@@ -173,66 +292,7 @@ __global__ void __launch_bounds__(64) k_nonbond_grid(BatchDev B, RunParams P) {
         const float4 plq = B.PLQs[I.a0 + i];
         e += (double)grid_sample(P.grid, pi, mk(plq.x, plq.y, plq.z), f);
     }
-    B.aforce[I.v0 + i] = make_float4(f.x, f.y, f.z, 0.f);
-    B.enb[I.a0 + i] = e;
-}
-
-// The same with a wave per atom, for batches with periodic molecules or substrate
-// atoms: their sums are long (atoms x images, thousands of terms with a root, an
-// exponential or a division each) and their batches small, so a thread per atom leaves
-// the card idle: 32 molecules of 40..96 atoms are 59 waves, each a chain of ~2000
-// terms.  A lane takes every 64th term, partners and images as one index; the 64
-// partial sums are added by a butterfly.  Those 32 molecules (9 images) take 36 us a step,
-// all launches included, instead of 259; 64 molecules of 16..128 atoms over a slab of
-// explicit atoms 34 instead of 66; the error against 64 bits falls from 6.6e-7 to 5.8e-7.
-// Batches with neither stay with the kernel above, whose partners come from LDS.
-// grid = (ceil(maxN/4), nsys), 256 threads; no barrier, a wave may end on its own.
-__global__ void __launch_bounds__(256) k_nonbond_lanes(BatchDev B, RunParams P) {
-    const int s = blockIdx.y;
-    if (B.status[s] != ST_RUNNING) return;
-    const SysInfo I = B.info[s];
-    const int N = I.natoms;
-    const int lane = threadIdx.x & 63;
-    const int i = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (i >= N) return;
-    const V3 pi = xyz(B.atoms[I.v0 + i]);
-    const float4 ri = B.REQs[I.a0 + i];
-    const float kQi = COULOMB_K * ri.z;
-    V3 f = zero3();
-    double e = 0.0;  // FP64 accumulation of the pair energies
-    if (P.bNonBonded && I.npbc > 0) {
-        nb_pbc_atom(B, I, i, pi, ri, lane, f, e);
-    } else if (P.bNonBonded) {
-        const unsigned* ex = B.excl + I.mask0 + i * ((N + 31) >> 5);
-        for (int j = lane; j < N; j += 64) {
-            const V3 d = xyz(B.atoms[I.v0 + j]) - pi;
-            const float4 rj = B.REQs[I.a0 + j];
-            if ((ex[j >> 5] >> (j & 31)) & 1u) continue;  // the atom itself among them
-            float fr, ep;
-            lj_pair<true, true>(d, ri.x + rj.x, ri.y * rj.y, kQi * rj.z, ri.w * rj.w, fr, ep);
-            f -= d * fr;
-            e += (double)ep;
-        }
-        for (int c = lane; c < I.ncorr; c += 64) {
-            const PairCorrDev pc = B.corr[I.corr0 + c];
-            if (pc.i != i) continue;
-            const V3 d = xyz(B.atoms[I.v0 + pc.j]) - pi;
-            const float4 rj = B.REQs[I.a0 + pc.j];
-            float fr, ep;
-            lj_pair<true, true>(d, ri.x + rj.x, ri.y * rj.y, kQi * rj.z, ri.w * rj.w, fr, ep);
-            f -= d * (fr * pc.w);
-            e += (double)ep * pc.w;
-        }
-    }
-    e *= 0.5;
-    if (P.nsurf > 0 && P.nsurf_pbc > 0) e += (double)surf_atoms_force(P, pi, ri, lane, f);
-    f = mk(wave_sum(f.x), wave_sum(f.y), wave_sum(f.z));
-    e = wave_sum_d(e);
-    if (P.bGridFF) {
-        const float4 plq = B.PLQs[I.a0 + i];
-        e += (double)grid_sample(P.grid, pi, mk(plq.x, plq.y, plq.z), f);
-    }
-    if (lane != 0) return;
+    if (P.nsurf > 0 && P.nsurf_pbc > 0) e += (double)surf_atoms_force<1>(P, pi, ri, 0, f);
     B.aforce[I.v0 + i] = make_float4(f.x, f.y, f.z, 0.f);
     B.enb[I.a0 + i] = e;
 }
@@ -573,11 +633,15 @@ __global__ void __launch_bounds__(256) k_precond(BatchDev B, RunParams P, float4
 }  // namespace fcd
 
 extern "C" hipError_t fc_launch_split_step(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P,
-                                           const int* node_sys, int ntot_nodes, int maxN, int do_move, int step) {
-    if (B->nperiodic > 0 || P->nsurf > 0)
-        hipLaunchKernelGGL(fcd::k_nonbond_lanes, dim3((maxN + 3) / 4, B->nsys), dim3(256), 0, st, *B, *P);
+                                           const fcd::NonbondPlan* nb, const int* node_sys, int ntot_nodes,
+                                           int do_move, int step) {
+    if (nb->tile_maxN > 0)
+        hipLaunchKernelGGL(fcd::k_nonbond_grid,
+                           dim3(nb->lane_n * nb->lane_maxN + (nb->tile_maxN + 63) / 64 * B->nsys), dim3(64), 0, st, *B,
+                           *P, *nb);
     else
-        hipLaunchKernelGGL(fcd::k_nonbond_grid, dim3((maxN + 63) / 64, B->nsys), dim3(64), 0, st, *B, *P);
+        hipLaunchKernelGGL(fcd::k_nonbond_lanes, dim3((nb->lane_maxN + 3) / 4, nb->lane_n), dim3(256), 0, st, *B, *P,
+                           *nb);
     hipLaunchKernelGGL(fcd::k_bonded, dim3((ntot_nodes + 255) / 256), dim3(256), 0, st, *B, *P, node_sys, ntot_nodes);
     hipLaunchKernelGGL(fcd::k_update, dim3(B->nsys), dim3(256), 0, st, *B, *P, do_move, step);
     return hipGetLastError();

@@ -24,7 +24,8 @@ extern "C" hipError_t fc_launch_zero_int(hipStream_t st, int* a, int n);
 extern "C" hipError_t fc_launch_zero_f4(hipStream_t st, float4* a, int n);
 extern "C" int fc_relax_lds_bytes(int nmax, int mmax, int block, int learned, int h2lds, int hb);
 extern "C" hipError_t fc_launch_split_step(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P,
-                                           const int* node_sys, int ntot_nodes, int maxN, int do_move, int step);
+                                           const fcd::NonbondPlan* nb, const int* node_sys, int ntot_nodes,
+                                           int do_move, int step);
 extern "C" hipError_t fc_launch_reset(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P);
 extern "C" hipError_t fc_launch_precond(hipStream_t st, const fcd::BatchDev* B, const fcd::RunParams* P, float4* out,
                                         const float* gnode, const float* gcomp);
@@ -246,13 +247,13 @@ void World::build_packed() {
     // image shifts: npbc per periodic system, one zero shift per vacuum system
     // (the reference's pbcshifts layout, nSys*npbc, for uniform batches)
     int nsh = 0;
-    n_periodic = 0;
+    pbc_sys.clear();
     for (int s = 0; s < nSys; s++) {
         const fc::MolSys& m = mols[s];
         info[s].sh0 = nsh;
         info[s].npbc = m.pbc ? (2 * m.nPBC[0] + 1) * (2 * m.nPBC[1] + 1) * (2 * m.nPBC[2] + 1) : 0;
         nsh += std::max(info[s].npbc, 1);
-        n_periodic += m.pbc ? 1 : 0;
+        if (m.pbc) pbc_sys.push_back(s);
     }
     pbcshifts.assign((size_t)nsh, f4(0, 0, 0, 0));
     nsteps.assign(nSys, 0);
@@ -470,6 +471,7 @@ bool World::upload_all(bool bParams, bool bForces, bool bVel) {
         d_bkNeighs.upload(bkNeighs, stream);
         d_neighCell.upload(neighCell, stream);
         d_pbcshifts.upload(pbcshifts, stream);
+        d_pbc_sys.upload(pbc_sys, stream);
         d_apars.upload(MMpars, stream);
         d_bLs.upload(BLs, stream);
         d_bKs.upload(BKs, stream);
@@ -588,13 +590,49 @@ fcd::BatchDev World::batch_dev() {
     B.sysflags = d_sysflags.p;
     B.gridcache = d_gridcache.p;
     B.pbcshifts = d_pbcshifts.p;
-    B.nperiodic = n_periodic;
     B.neighCell = d_neighCell.p;
     B.snap = (snap_on && d_snap.p) ? d_snap.p : nullptr;
     B.snap_every = std::max(snap_every, 1);
     B.nsnap = nsnap;
     B.ntotV = ntotV;
     return B;
+}
+
+// Non-bonded kernels of a split step over all systems, or over those of todo.  Periodic
+// molecules take a wave per atom at every size (k_nonbond_lanes).  A vacuum molecule takes a
+// thread per atom, as in batches of vacuum molecules alone, unless the step has images or
+// substrate atoms to sum and a wave per atom is through the batch before a thread is
+// through the longest chain: iterations of 64 terms and 3 for the sums of every atom, about
+// 6000 a us on the full card, against 0.13 us for each term of the chain, 1536 workgroups
+// of 64 threads at a time.  A step with a wave and with a thread per atom took, in us:
+//   one periodic molecule among 128 / 1024 of 16..256 atoms      34, 62 / 119, 78
+//   the same over the grid, among 128                            39, 64
+//   512 molecules of 16..128 atoms over 8 x 25 substrate atoms   62, 57
+//   512 / 4096 of 8..24 atoms over 8 x 25                        29, 48 / 85, 85
+//   512 / 2048 of 16..128 atoms over 8 x 1                       48, 38 / 144, 66
+fcd::NonbondPlan World::nonbond_plan(const std::vector<int>* todo, const int* dev_todo) const {
+    if (pbc_sys.empty() && surf_pos.empty()) return {nullptr, 0, 0, maxN};
+    const int n = todo ? (int)todo->size() : nSys;
+    double atoms = 0, pairs = 0, tiles = 0;  // of the vacuum molecules
+    int vac = 0, pbc = 0;                    // the largest
+    for (int k = 0; k < n; k++) {
+        const fcd::SysInfo& I = info[todo ? (*todo)[k] : k];
+        const int N = I.natoms;
+        if (I.npbc > 0) {
+            pbc = std::max(pbc, N);
+            continue;
+        }
+        vac = std::max(vac, N);
+        atoms += N;
+        pairs += (double)N * N;
+        tiles += (N + 63) / 64;
+    }
+    const int npbc = (int)pbc_sys.size();
+    if (vac == 0) return {npbc < nSys ? d_pbc_sys.p : nullptr, npbc, pbc, 0};
+    const double terms = (double)surf_pos.size() * surf_shifts.size();
+    if (pairs + atoms * (terms + 192) < 5e4 * (vac + terms) * std::max(1.0, tiles / 1536))
+        return {dev_todo, n, std::max(vac, pbc), 0};
+    return {d_pbc_sys.p, npbc, pbc, vac};
 }
 
 fcd::RunParams World::run_params(double Fconv, int nstep_max) {
@@ -1010,9 +1048,14 @@ bool World::scan(int nconf, const double* poss, const double* rots, double* Es, 
 // FIRE on the exact force: the other systems keep their final state and are
 // skipped.  Adds the device time to last_ms.
 bool World::relax_unclassed(int nstep_max, double Fconv) {
-    std::vector<int> only(nSys, 0);
-    for (int s = 0; s < nSys; s++) only[s] = (sys_class[s] < 0) ? 1 : 0;
+    std::vector<int> only(nSys, 0), todo;
+    for (int s = 0; s < nSys; s++) {
+        only[s] = (sys_class[s] < 0) ? 1 : 0;
+        if (only[s]) todo.push_back(s);
+    }
     d_only.upload(only, stream);
+    d_todo.upload(todo, stream);
+    const fcd::NonbondPlan nb = nonbond_plan(&todo, d_todo.p);
     fcd::BatchDev B = batch_dev();
     fcd::RunParams P = run_params(Fconv, nstep_max);
     P.pc_mode = 0;
@@ -1024,7 +1067,7 @@ bool World::relax_unclassed(int nstep_max, double Fconv) {
     for (int step = 0; step <= nstep_max;) {
         const int n = std::min(chunk, nstep_max + 1 - step);
         for (int k = 0; k < n; k++, step++)
-            if (!hip_ok(fc_launch_split_step(stream, &B, &P, d_node_sys.p, ntotM, maxN, 1, step), "split step"))
+            if (!hip_ok(fc_launch_split_step(stream, &B, &P, &nb, d_node_sys.p, ntotM, 1, step), "split step"))
                 return false;
         d_status.download(status, stream);
         if (!hip_ok(hipStreamSynchronize(stream), "split status")) return false;
@@ -1047,6 +1090,7 @@ int World::relax_split(int nstep_max, double Fconv, bool restore_start) {
                "restore");
     fcd::BatchDev B = batch_dev();
     fcd::RunParams P = run_params(Fconv, nstep_max);
+    const fcd::NonbondPlan nb = nonbond_plan();
     hipMemsetAsync(d_avel.p, 0, sizeof(float4) * ntotV, stream);
     fc_launch_zero_f4(stream, d_stall.p, nSys);  // no learned form here: no fallback flags
     fc_launch_reset(stream, &B, &P);
@@ -1058,7 +1102,7 @@ int World::relax_split(int nstep_max, double Fconv, bool restore_start) {
     for (; step <= nstep_max;) {
         int n = std::min(chunk, nstep_max + 1 - step);
         for (int k = 0; k < n; k++, step++)
-            if (!hip_ok(fc_launch_split_step(stream, &B, &P, d_node_sys.p, ntotM, maxN, 1, step), "split step"))
+            if (!hip_ok(fc_launch_split_step(stream, &B, &P, &nb, d_node_sys.p, ntotM, 1, step), "split step"))
                 return -1;
         d_status.download(status, stream);
         hip_ok(hipStreamSynchronize(stream), "split status");
@@ -1115,13 +1159,14 @@ int World::explore(int nstep_max, double Fconv, double T, double gamma, int n_ex
     P.xn_relax = std::max(n_relax, 0);
     P.xseed = seed;
     P.xkmax = kmax;
+    const fcd::NonbondPlan nb = nonbond_plan();
     hipMemsetAsync(d_avel.p, 0, sizeof(float4) * ntotV, stream);
     fc_launch_reset(stream, &B, &P);
     EventSet events;
     hipEvent_t e0 = events.make(), e1 = events.make();
     hipEventRecord(e0, stream);
     for (int step = 0; step <= nstep_max; step++)
-        if (!hip_ok(fc_launch_split_step(stream, &B, &P, d_node_sys.p, ntotM, maxN, 1, step), "explore step"))
+        if (!hip_ok(fc_launch_split_step(stream, &B, &P, &nb, d_node_sys.p, ntotM, 1, step), "explore step"))
             return -1;
     hipEventRecord(e1, stream);
     // DevArr::download fills the host vector's current size: size them first
@@ -1174,8 +1219,9 @@ bool World::eval_forces() {
     if (!dev_ready || nSys == 0) return false;
     fcd::BatchDev B = batch_dev();
     fcd::RunParams P = run_params(0.0, 0);
+    const fcd::NonbondPlan nb = nonbond_plan();
     fc_launch_reset(stream, &B, &P);
-    if (!hip_ok(fc_launch_split_step(stream, &B, &P, d_node_sys.p, ntotM, maxN, 0, 0), "eval_forces")) return false;
+    if (!hip_ok(fc_launch_split_step(stream, &B, &P, &nb, d_node_sys.p, ntotM, 0, 0), "eval_forces")) return false;
     return hip_ok(hipStreamSynchronize(stream), "eval_forces sync");
 }
 

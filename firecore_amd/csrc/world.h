@@ -156,7 +156,7 @@ struct World {
         d_fire, d_stall, d_grid;
     DevArr<int4> d_neighs, d_bkNeighs, d_neighCell;
     DevArr<float4> d_pbcshifts;
-    int n_periodic = 0;  // periodic molecules in the batch (relaxed by the split kernels)
+    std::vector<int> pbc_sys;  // periodic molecules of the batch (relaxed by the split kernels)
     int nPBC_init[3] = {0, 0, 0};  // image range given to init()
     // lattice (rows a, b, c) and image range of system isys (all if < 0); lvec
     // null makes it a vacuum molecule again.  Re-packs and uploads the batch.
@@ -173,7 +173,7 @@ struct World {
     int n_unclassed = 0;  // systems too large for every class (relaxed by the split kernels)
     bool record_times = false;  // per-system start/end wall clock of the persistent kernel
     DevArr<long long> d_systime;
-    DevArr<int> d_only;
+    DevArr<int> d_only, d_pbc_sys, d_todo;
     bool hb_batch = false;
     bool autotune = true;
     // cost estimate of a system for the queue order (longest first):
@@ -205,6 +205,8 @@ struct World {
     bool set_grid(const fc::GridFFHost& g);
     void register_buffers();
     fcd::BatchDev batch_dev();
+    // todo: the systems to be worked on (null: all), in device memory at dev_todo
+    fcd::NonbondPlan nonbond_plan(const std::vector<int>* todo = nullptr, const int* dev_todo = nullptr) const;
     fcd::RunParams run_params(double Fconv, int nstep_max);
     // launch plan of the persistent kernel; upload = false leaves the queue
     // order in h_order only (the allocation-free path copies it itself)
