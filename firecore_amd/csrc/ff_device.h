@@ -51,15 +51,19 @@ __device__ __forceinline__ float dpp_shl1_zero(float src) {
                                                                  true));
 }
 
-// Stores v at LDS byte address `addr` + off (off a constant) from lane 0 alone;
-// all lanes call with exec full.  Narrowing exec for one instruction costs two
-// scalar ones; the branch the compiler makes of `if (lane == 0)` costs six and
-// splits the block, so nothing is scheduled across it.
+// Stores v at LDS byte address `addr` + off (off a constant) from lane 0 alone, if it is
+// active.  Narrowing exec for one instruction costs two scalar ones; the branch the compiler
+// makes of `if (lane == 0)` costs six and splits the block, so nothing is scheduled across
+// it.  exec comes back as it was.
 typedef float f32x3 __attribute__((ext_vector_type(3)));
-#define lane0_store(addr, off, v)                                                                          \
-    asm volatile("s_mov_b64 exec, 1\n\tds_write_b96 %0, %1 offset:%2\n\ts_mov_b64 exec, -1" ::"v"(addr), \
-                 "v"(f32x3{(v).x, (v).y, (v).z}), "n"(off)                                                 \
-                 : "memory")
+#define lane0_store(addr, off, v)                                                                               \
+    do {                                                                                                        \
+        unsigned long long saved_;                                                                              \
+        asm volatile("s_and_saveexec_b64 %0, 1\n\tds_write_b96 %1, %2 offset:%3\n\ts_mov_b64 exec, %0"          \
+                     : "=&s"(saved_)                                                                            \
+                     : "v"(addr), "v"(f32x3{(v).x, (v).y, (v).z}), "n"(off)                                     \
+                     : "memory", "scc");                                                                        \
+    } while (0)
 
 // All ones where bit BIT of w is set, else 0 (one instruction; as C++ the and
 // with it becomes an and, a compare and a select).

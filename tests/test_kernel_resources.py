@@ -1,6 +1,7 @@
 """The build refuses a kernel with register spills: one instance of the relaxation kernel
 that spilled has faulted the GPU (the spill was stored with the execution mask still off)."""
 import os
+import re
 
 import pytest
 
@@ -37,3 +38,11 @@ def test_built_kernels_have_no_scratch():
     res = fb.resources()
     assert sum("relax_persistent_kernel" in k for k in res) == 32
     fb.check_scratch(res)
+
+
+def test_inline_assembly_restores_the_execution_mask():
+    """Assembly that narrows exec puts back what it found: a constant would turn on the lanes
+    of a caller in divergent code."""
+    for name in os.listdir(fb.CSRC):
+        with open(os.path.join(fb.CSRC, name)) as f:
+            assert not re.search(r"exec(_lo|_hi)?, *-?\d", f.read()), name
