@@ -1054,8 +1054,9 @@ bool World::relax_unclassed(int nstep_max, double Fconv) {
         if (only[s]) todo.push_back(s);
     }
     d_only.upload(only, stream);
-    d_todo.upload(todo, stream);
-    const fcd::NonbondPlan nb = nonbond_plan(&todo, d_todo.p);
+    const bool all = (int)todo.size() == nSys;
+    if (!all) d_todo.upload(todo, stream);
+    const fcd::NonbondPlan nb = all ? nonbond_plan() : nonbond_plan(&todo, d_todo.p);
     fcd::BatchDev B = batch_dev();
     fcd::RunParams P = run_params(Fconv, nstep_max);
     P.pc_mode = 0;
