@@ -1276,7 +1276,7 @@ int train_proposal(int iters, double lr, double eta, double dmax, long long seed
 // 2 = evaluate the proposal network inside the persistent relaxation kernel
 // with its second activation buffer in global memory (default; leaves the
 // kernel's LDS footprint, and so its occupancy, unchanged), 1 = the same with
-// that buffer in LDS where the class's LDS budget allows, 0 = chunked
+// that buffer in LDS where it costs the class no resident workgroup, 0 = chunked
 // relaunches with a separate network kernel between chunks (graph replay).
 // Returns the previous setting.
 int set_learned_inkernel(int on) {

@@ -74,6 +74,25 @@ def test_residency_of_plain_rows(lib, static, block):
     assert not less, (len(less), less[:3])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("natoms,block", [(20, 64), (44, 64), (61, 64), (64, 64), (122, 128), (126, 128), (190, 192),
+                                          (248, 256), (251, 256)])
+def test_second_activation_buffer_costs_no_workgroup(static, natoms, block):
+    lds = {}
+    try:
+        native.set_proposal_weights(np.load("firecore_amd/proposal_weights.npy"))
+        for mode in (2, 1):
+            native.set_learned_inkernel(mode)
+            native.set_precond(2, 3.0, 127.0)
+            native.init_workload(0, 1, 0, natoms, natoms, 0.1, None, 0.1)
+            lds[mode], = [c["lds"] for c in native.class_info() if c["block"] == block]
+    finally:
+        native.set_learned_inkernel(2)
+        native.set_precond(0)
+    st = static(block, 0, "learned")
+    assert per_cu(block, lds[1], st) >= per_cu(block, lds[2], st), lds
+
+
 @pytest.mark.parametrize("learned,h2lds,hb", [(0, 0, 0), (0, 0, 1), (1, 0, 0), (1, 0, 1), (1, 1, 0), (1, 1, 1)])
 def test_arrays_do_not_overlap(lib, learned, h2lds, hb):
     names = ["pos", "pi", "fnb", "re", "hb", "facc", "fself", "fng", "mask", "h", "nb", "gain", "h2", "end"]
