@@ -178,7 +178,10 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
         const int N = I.natoms, M = I.nnode, V = N + M;
         const int sflags = B.sysflags ? B.sysflags[s] : 0;  // restraints (bit 0), walls (bit 1)
         const int W = (N + 31) >> 5;   // exclusion words per atom in memory
-        const int Kl = N >> 1;         // last offset of the half ring
+        // last offset of the half ring; without non-bonded terms 0, which leaves one masked
+        // iteration of the pair loop, for the grid window's halves, and none in vacuum: all
+        // offsets masked took 68 us a step for 4096 vacuum systems of 16..256 atoms, this 22
+        const int Kl = P.bNonBonded ? N >> 1 : 0;
         const int Wh = Kl >> 5;        // its exclusion word, kept in a register; the words below it are in LDS
         const int PR = LdsLayout::prow_of(N);  // periodic rows of this system
         // exclusion rows transposed to [word][atom] so that lanes read consecutive banks
@@ -393,7 +396,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                     float4* slots = B.gridcache + (size_t)(I.a0 + wu * 64) * 16;
                     const int nslot = min(64, N - wu * 64);
                     if (onGrid) gw.refill(P.grid, lane, plq, slots, nslot);
-                    if (wu < nwAct && (P.bNonBonded || onGrid)) {
+                    if (wu < nwAct && (Kl > 0 || onGrid)) {
                         const int ia = hasAtom ? tid : 0;
                         const float4* pp = s_pos + ia;
                         const float2* pr = s_re + ia;
@@ -438,10 +441,7 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                         a0 = rows(0);
                         a1 = rows(1);
                         unsigned keep = 0;
-                        // offsets taken: 0..Kn-1.  Without non-bonded terms one masked iteration,
-                        // for the window's halves, and no loop at all in vacuum: all offsets masked
-                        // took 68 us a step for 4096 vacuum systems of 16..256 atoms, this 22.
-                        const int Kn = P.bNonBonded ? (Kl & ~3) + 4 : 4;
+                        const int Kn = (Kl & ~3) + 4;  // offsets taken: 0..Kn-1
                         const int kmid = (Kn >> 3) << 2;
                         if (onGrid) gw.fetch(hasAtom ? lane : 0, slots, nslot, 0);
                         else gw.no_fetch();
@@ -455,7 +455,6 @@ relax_persistent_kernel(BatchDev B, RunParams P, Queues Q, int cls,
                                 const int w = k >> 5;
                                 keep = ~(w < Wh ? s_mask[w * N + ia] : mlast);
                                 if (w == 0) keep &= ~1u;
-                                if (!P.bNonBonded) keep = 0;
                                 if (w == Wh) {  // nothing past N/2; for even N the pair at N/2 is the lower half's
                                     const int top = (Kl & 31) + ((!(N & 1) && tid >= Kl) ? 0 : 1);
                                     keep &= top < 32 ? (1u << top) - 1u : ~0u;
