@@ -316,8 +316,8 @@ __device__ __forceinline__ void mlp_forward(const MlpDev& M, unsigned short* h, 
 // Forward pass used by the relaxation kernel between segments of its step
 // loop (nothing of the force loop is live there, so a layer may hold all its
 // weight fragments in registers).  Activations alternate between two
-// row buffers of n rows, hA (LDS) and hG (LDS when the workgroup's LDS budget
-// allows, else a per-workgroup slot in global memory that stays in L2):
+// row buffers of n rows, hA (LDS) and hG (LDS when that costs no resident
+// workgroup, else a per-workgroup slot in global memory that stays in L2):
 // layer 1 hA -> hG, layer 2 hG -> hA, layer 3 hA -> hG, head from hG.
 template <int BLOCK, int KIN, class NB>
 __device__ __forceinline__ void mlp_layer_rows(const unsigned short* hin, const NB* nb, const unsigned short* W,

@@ -353,7 +353,7 @@ int proposal_backward(const float* dout, float* grad);
 /* Adam training on the recorded snapshots, one snapshot per system per step */
 int train_proposal(int iters, double lr, double eta, double dmax, long long seed, float* loss_hist);
 /* 2 = proposal network inside the persistent kernel, activations spill to global (default);
- * 1 = the same with LDS activations where the LDS budget allows; 0 = chunked relaunches */
+ * 1 = the same with LDS activations where that costs no resident workgroup; 0 = chunked relaunches */
 int set_learned_inkernel(int on);
 /* chunk iterations of the last learned relaxation */
 int get_last_chunks(void);
